@@ -303,7 +303,7 @@ int run_qmm(imq_ctx* ctx, const char* fn, Regime regime, const uint32_t* w, cons
 namespace {
 
 // Shared checks of the fused-epilogue entry points: the qmm checks, then T in
-// {bf16, f16} (any K % 64 == 0: K % 256 != 0 runs the register-staged tile
+// {bf16, f16} (any K % 64 == 0: a short ragged K runs the register-staged tile
 // kernel with the same output stage).
 int check_epilogue(imq_ctx* ctx, const char* fn, const uint32_t* w, const void* s, const void* b,
                    const void* x, const void* y, int k, int n, int m, int group_size, int bits,

@@ -87,7 +87,8 @@ struct QgemmPlan {
 QgemmPlan qgemm_plan(int k, int n, int m, bool fused, bool split, int cus, bool pair = false);
 
 // Whether the buffer-load MFMA kernel (and so the fused epilogues) takes
-// these shapes: K % 256 == 0 and x, w addressable with 32-bit byte offsets.
+// these shapes: x and w addressable with 32-bit byte offsets, K % 64 == 0 but
+// for a short ragged K (K % 256 != 0), which is the register-staged kernel's.
 bool qgemm_big_supported(int k, int n, int m);
 
 // Fused output stages on the MFMA kernels (T in {bf16, f16}; any K % 64 == 0:

@@ -1,0 +1,55 @@
+// qgemm_plan.hpp -- what qgemm.hip (plans, dispatch) and the translation units
+// that hold the tile kernels (qgemm_tile.hpp) share.
+#pragma once
+
+#include <type_traits>
+
+#include "epilogue.hpp"
+#include "imq_kernels.hpp"
+
+namespace imq {
+
+// Tile height (32 mt rows), width (128 nt columns) and K split of a launch of
+// the large-M kernel; split_steps K-steps of 128 per split, an even
+// number (K % 256 == 0) or all of them.
+struct BigPlan {
+  int mt, nt, splits, split_steps;
+};
+
+namespace tile {
+
+// The register-staged kernel with output stage ep (any K % 64 == 0).
+template <int T, class EP>
+hipError_t launch_reg(const uint32_t* w, const uint16_t* scales, const uint16_t* biases,
+                      const uint16_t* x, const EP& ep, int k, int n, int m, hipStream_t stream);
+// The large-M kernel by plan p, with output stage ep or (EpPartial) the
+// partial sums of p.splits K ranges.  KT: K % 256 != 0.
+template <int T, class EP, bool KT>
+hipError_t launch_plan(const BigPlan& p, const uint32_t* w, const uint16_t* scales,
+                       const uint16_t* biases, const uint16_t* x, const EP& ep, int k, int n,
+                       int m, hipStream_t stream);
+// The sum of a split launch's partial sums with output stage ep.
+template <int T, class EP>
+hipError_t launch_sum(const SplitWs& ws, int splits, int m, int ncols, int ldp, const EP& ep,
+                      hipStream_t stream);
+
+// Stages built for every tile height and for 128-column tiles: the plain
+// store, the split-K partial sums and the text encoder's residual add; the
+// other fused stages are built for 128 rows and more.
+template <int T, class EP>
+constexpr bool kAnyTile = EP::kPartial || (!EP::kPair && (std::is_same<EP, EpStore<T>>::value ||
+                                                          std::is_same<EP, EpResidAdd<T>>::value));
+
+// Tiles built for stage EP (mt: 32-row units, nt: 128-column units).
+template <int T, class EP, bool KT>
+constexpr bool tile_built(int mt, int nt) {
+  if (nt == 1 && (EP::kPair || !kAnyTile<T, EP>)) return false;
+  if (mt < 4 && !kAnyTile<T, EP>) return false;
+  // K % 256 != 0: fewer heights (the planner's list is the same).
+  if (KT) return nt == 1 ? (mt == 2 || mt == 4) : (mt != 5 && mt != 7);
+  return true;
+}
+
+}  // namespace tile
+
+}  // namespace imq
