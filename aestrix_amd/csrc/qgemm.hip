@@ -10,40 +10,55 @@
 namespace imq {
 namespace {
 
-// Tile height, width and K split of the large-M kernel (small: 32- and 64-row
-// and 128-column tiles allowed without a split -- the plain store and the
-// residual add are built for them, the other fused stages are not, the
-// split-K partial sums always are; split: K may be split).  Cost in units of about
-// 0.36 us (a K-step of a 32-row slice of the tile): a round of tiles costs
-// split_steps * (MT + 1.5) plus 12 for its prologue and output; a split adds
-// the workspace traffic of its reduction (8 bytes per output and split, at
-// about 1.4 MB per unit) plus 3 for the extra launch.  Splits are taken only
-// when the tiles leave CUs idle.  160-row tiles exist for row counts that
-// leave a round of 192-row tiles part empty: 1024 x 9216 at K = 3072 is 252
-// tiles in one round instead of 216 (58.4 -> 57.0 us), 2048 x 9216 is 468
-// tiles in two rounds instead of 396 in two (115.0 -> 105.6 us).
+// What a launch costs, in one unit per model: a round of tiles
+// split_steps * step(mt, nt) plus its prologue and output, a split its second
+// launch and the workspace traffic (per output and split).
 //
-// 128-column tiles (one 32-column tile per wave, NT = 1) double the tiles of
-// a shape at a given height, so a short M keeps a taller tile.  What bounds a
-// K-step of a 32- or 64-row tile is its dequant VALU work, the same per wave
-// and weight fragment at any height (each fragment feeds MT MFMAs), not its
-// MFMAs: half the columns per wave halve it.  Cost of a NT = 1 step:
-// max(kNt1Floor, kNt1Step + kNt1PerRow * MT), fitted to forced plans timed on
-// the text-encoder and DiT shapes (M = 128-2048, same box: e.g. M = 512 K =
-// 2560 N = 6144 at 128 x 128 tiles 18.8 us against 21.5 at 64 x 256; N = 2560
-// K = 4096 unsplit at 64 x 128 20.0 against 23.4 split three ways at 64 x
-// 256).  The narrower tiles read 1.5x the activation and weight bytes per
-// flop of 256-column ones from L2: they are taken only where a split's
-// activation panel (M rows x its K range) fits one XCD's 4 MB L2 (at M = 512
-// K = 9216 unsplit 64 x 128 tiles ran at 57.6 us against 42.0 for 128 x 256
-// tiles split four ways), and a split of them is costed 3 units more.  Only
-// for stages other than a gate/up pair (whose wave holds gate and up
-// columns), unsplit only for the plain store.
-constexpr double kNt1Floor = 1.5, kNt1Step = -0.35, kNt1PerRow = 0.925;
-constexpr size_t kNt1MaxPanel = (size_t)4 << 20;
-BigPlan pick_big_plan(int m, int n, int k, int cus, bool small, bool split, bool pair = false) {
+// 128-column tiles (one 32-column tile per wave, nt = 1) double the tiles of a
+// shape at a given height, so a short M keeps a taller tile (each dequantized
+// weight fragment feeds mt MFMAs); they read 1.5x the activation and weight
+// bytes per flop of 256-column ones.
+//
+// kFit (us): fitted to 2300 forced plans (every tile, up to 12 splits, on 75
+// shapes of 33 to 4608 rows, weights past the last-level cache): its pick is
+// 0.5% slower than the fastest plan on average and 6.5% at worst, where the
+// former model's was 3.4% and 33% slower.  The former model (units of about
+// 0.36 us) kept 128-column tiles to activation panels under 4 MB and costed a
+// split's second launch at a fifth: [1024 x 3072] K = 3072 28.4 us on 64 x 256
+// tiles against 23.6 on 128 x 128, [1300 x 1536] K = 4096 31.9 (32 x 256)
+// against 24.6 (64 x 128), [3000 x 2048] K = 6144 81.1 (192 x 256 split in
+// two) against 70.3 (192 x 128 unsplit).  It stays for outputs whose partial
+// sums of even two splits outgrow the static scratch (8.4 M outputs): there
+// both pick alike, and the shapes that the allocation-free entry refuses stay
+// the same; and for launches that share the CUs with another stream's (shared),
+// whose 256-column tiles leave the L2 to both: a denoise step of 1512 + 512
+// rows 1633 us with it, 1661 with kFit.  Below that size a split's partial sums fit that scratch.
+struct CostModel {
+  double step2[9], step1[9];  // per K-step, by mt: 256 and 128 columns
+  double round2, round1;      // per round of tiles
+  double split2, split1;      // per split launch
+  double per_split;           // and per split of it
+  double per_output;          // per output and split
+};
+constexpr CostModel kFit = {
+    {0, 0.782, 0.967, 0, 1.477, 1.767, 2.102, 2.449, 2.614},
+    {0, 0, 0.557, 0, 0.840, 0.978, 1.211, 1.398, 1.512},
+    3.878, 2.818, 2.975, 2.975, 0.371, 1.11e-6};
+constexpr CostModel kLarge = {
+    {0, 2.5, 3.5, 0, 5.5, 6.5, 7.5, 8.5, 9.5},
+    {0, 0, 1.5, 0, 3.35, 4.275, 5.2, 6.125, 7.05},
+    12.0, 12.0, 3.0, 6.0, 0.0, 8.0 / 1.4e6};
+constexpr size_t kLargeMaxPanel = (size_t)4 << 20;  // of a 128-column tile's activations
+
+// Tile and K split of a launch over n weight rows (split: K may be split;
+// pair: a gate/up pair, whose wave holds gate and up columns: 256-column tiles
+// of 128 rows and more).  Splits are taken only when the tiles leave CUs idle.
+BigPlan pick_big_plan(int m, int n, int k, int cus, bool split, bool pair = false,
+                      bool shared = false) {
   const int steps = (k + 255) / 256 * 2;  // of 128, whole scale blocks
   const bool tail = k % 256 != 0;
+  const bool large = shared || (size_t)m * n * 8 > kStaticScratchBytes;
+  const CostModel& c = large ? kLarge : kFit;
   BigPlan best{8, 2, 1, steps};
   double best_cost = 1e30;
   for (int nt : {2, 1}) {
@@ -57,21 +72,22 @@ BigPlan pick_big_plan(int m, int n, int k, int cus, bool small, bool split, bool
       // K % 256 != 0 is built for fewer tiles (tile::tile_built).
       if (tail && (nt == 1 ? mt > 4 : mt == 5 || mt == 7)) continue;
       const long tiles = (long)((m + 32 * mt - 1) / (32 * mt)) * tiles_n;
-      const int max_splits = split && tiles < cus ? std::max(1, steps / 2) : 1;
+      // Up to two rounds of workgroups (the former model: any).
+      const int max_splits =
+          !split || tiles >= cus ? 1
+          : large                ? std::max(1, steps / 2)
+                                 : std::max(1, (int)std::min<long>(steps / 2, 2 * cus / tiles));
       for (int sp = 1; sp <= max_splits; ++sp) {
         const int sps = ((steps + sp - 1) / sp + 1) / 2 * 2;  // even
         const int eff = (steps + sps - 1) / sps;
-        if (eff != sp || (eff == 1 && mt < 4 && !small)) continue;
-        // With K % 256 != 0 a split's partial sums stay within the static
-        // scratch, so that the allocation-free entry takes every such shape.
-        if (tail && eff > 1 && (size_t)eff * m * n * 4 > kStaticScratchBytes) continue;
-        if (nt == 1 && ((eff == 1 && !small) || (size_t)m * sps * 128 * 2 > kNt1MaxPanel))
-          continue;
+        if (eff != sp || (eff == 1 && mt < 4 && pair)) continue;
+        if ((!large || tail) && eff > 1 && (size_t)eff * m * n * 4 > kStaticScratchBytes) break;
+        if (large && nt == 1 && (size_t)m * sps * 128 * 2 > kLargeMaxPanel) continue;
         const long rounds = (tiles * eff + cus - 1) / cus;
-        const double step =
-            nt == 2 ? mt + 1.5 : std::max(kNt1Floor, kNt1Step + kNt1PerRow * mt);
-        double cost = (double)rounds * (sps * step + 12.0);
-        if (eff > 1) cost += (double)eff * m * n * 8.0 / 1.4e6 + (nt == 2 ? 3.0 : 6.0);
+        double cost = (double)rounds *
+                      (sps * (nt == 2 ? c.step2[mt] : c.step1[mt]) + (nt == 2 ? c.round2 : c.round1));
+        if (eff > 1)
+          cost += (nt == 2 ? c.split2 : c.split1) + eff * (c.per_split + (double)m * n * c.per_output);
         if (cost < best_cost - 1e-9) {
           best_cost = cost;
           best = BigPlan{mt, nt, eff, sps};
@@ -126,7 +142,6 @@ hipError_t launch_big_ep(const uint32_t* w, const uint16_t* scales, const uint16
   // offsets: the register-staged kernel, one pass.
   if (!qgemm_big_supported(k, n, m))
     return tile::launch_reg<T, EP>(w, scales, biases, x, ep, k, n, m, stream);
-  constexpr bool kSmall = tile::kAnyTile<T, EP>;
   int cols = n;  // weight rows covered
   int width = n, gate_row = 0, up_row = 0;
   if constexpr (EP::kPair) {
@@ -137,9 +152,9 @@ hipError_t launch_big_ep(const uint32_t* w, const uint16_t* scales, const uint16
   }
   const bool tail = k % 256 != 0;
   const int cus = ws.cus > 0 ? ws.cus : device_cus();
-  BigPlan p = pick_big_plan(m, cols, k, cus, kSmall, ws.p != nullptr, EP::kPair);
+  BigPlan p = pick_big_plan(m, cols, k, cus, ws.p != nullptr, EP::kPair, ws.cus > 0);
   if (p.splits > 1 && ws.bytes < (size_t)p.splits * m * cols * sizeof(float))
-    p = pick_big_plan(m, cols, k, cus, kSmall, false, EP::kPair);  // no room for the partial sums
+    p = pick_big_plan(m, cols, k, cus, false, EP::kPair, ws.cus > 0);  // no room for the partial sums
   if (p.splits == 1)
     return tail ? tile::launch_plan<T, EP, true>(p, w, scales, biases, x, ep, k, n, m, stream)
                 : tile::launch_plan<T, EP, false>(p, w, scales, biases, x, ep, k, n, m, stream);
@@ -184,19 +199,18 @@ hipError_t launch_qgemm(const uint32_t* w, const void* scales, const void* biase
 size_t qgemm_split_bytes(int k, int n, int m, bool fused) {
   if (!qgemm_big_supported(k, n, m)) return 0;
   // The most a stage over these rows takes: a fused stage may be a gate/up
-  // pair (no 128-column tiles), the residual add (every tile) or another.
+  // pair (no 128-column tiles) or another.
   size_t bytes = 0;
-  for (int v = 0; v < (fused ? 3 : 1); ++v) {
-    const bool small = !fused || v == 2, pair = v == 1;
-    const BigPlan p = pick_big_plan(m, n, k, device_cus(), small, true, pair);
+  for (int v = 0; v < (fused ? 2 : 1); ++v) {
+    const BigPlan p = pick_big_plan(m, n, k, device_cus(), true, v == 1);
     if (p.splits > 1) bytes = std::max(bytes, (size_t)p.splits * m * n * sizeof(float));
   }
   return bytes;
 }
 
-QgemmPlan qgemm_plan(int k, int n, int m, bool fused, bool split, int cus, bool pair) {
+QgemmPlan qgemm_plan(int k, int n, int m, bool, bool split, int cus, bool pair) {
   if (!qgemm_big_supported(k, n, m)) return QgemmPlan{false, 128, 1, 0, 256};
-  const BigPlan p = pick_big_plan(m, n, k, cus > 0 ? cus : device_cus(), !fused, split, pair);
+  const BigPlan p = pick_big_plan(m, n, k, cus > 0 ? cus : device_cus(), split, pair);
   return QgemmPlan{true, 32 * p.mt, p.splits,
                    p.splits > 1 ? (size_t)p.splits * m * n * sizeof(float) : 0, 128 * p.nt};
 }

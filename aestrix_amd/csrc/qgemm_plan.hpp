@@ -2,8 +2,6 @@
 // that hold the tile kernels (qgemm_tile.hpp) share.
 #pragma once
 
-#include <type_traits>
-
 #include "epilogue.hpp"
 #include "imq_kernels.hpp"
 
@@ -33,18 +31,11 @@ template <int T, class EP>
 hipError_t launch_sum(const SplitWs& ws, int splits, int m, int ncols, int ldp, const EP& ep,
                       hipStream_t stream);
 
-// Stages built for every tile height and for 128-column tiles: the plain
-// store, the split-K partial sums and the text encoder's residual add; the
-// other fused stages are built for 128 rows and more.
-template <int T, class EP>
-constexpr bool kAnyTile = EP::kPartial || (!EP::kPair && (std::is_same<EP, EpStore<T>>::value ||
-                                                          std::is_same<EP, EpResidAdd<T>>::value));
-
 // Tiles built for stage EP (mt: 32-row units, nt: 128-column units).
 template <int T, class EP, bool KT>
 constexpr bool tile_built(int mt, int nt) {
-  if (nt == 1 && (EP::kPair || !kAnyTile<T, EP>)) return false;
-  if (mt < 4 && !kAnyTile<T, EP>) return false;
+  // A gate/up pair: 256 columns and 128 rows or more; its partial sums any height.
+  if (EP::kPair && (nt == 1 || (mt < 4 && !EP::kPartial))) return false;
   // K % 256 != 0: fewer heights (the planner's list is the same).
   if (KT) return nt == 1 ? (mt == 2 || mt == 4) : (mt != 5 && mt != 7);
   return true;

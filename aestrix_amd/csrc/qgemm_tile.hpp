@@ -985,8 +985,8 @@ hipError_t launch_big(const BigPlan& p, const uint32_t* w, const uint16_t* scale
 // the output stage ep (its T rounding of value / value2, then emit8 or
 // emit1): 8 consecutive outputs of a row per thread.  Partials of split s
 // sit at ws + s * M * ldp; plain stages read column c at c, pair stages the
-// gate sum at c and the up sum at width + c.  vload: ldp % 4 == 0 and
-// ncols % 8 == 0 (16-byte partial loads).
+// gate sum at c and the up sum at width + c.  vload: every row and pair offset
+// allows 16-byte partial loads.
 template <int T, class EP>
 __global__ __launch_bounds__(256) void reduce_ep_kernel(const float* __restrict__ ws, int splits,
                                                         int M, int ncols, int ldp, bool vload,
@@ -1000,7 +1000,7 @@ __global__ __launch_bounds__(256) void reduce_ep_kernel(const float* __restrict_
   float a[8], u[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) a[e] = u[e] = 0.f;
-  if (vload) {
+  if (vload && c0 + 8 <= ncols) {
     // The loads of kBatch splits go out before the first add (indices past
     // the last split repeat it and are not added): one memory round trip per
     // batch instead of one per split.
@@ -1029,14 +1029,30 @@ __global__ __launch_bounds__(256) void reduce_ep_kernel(const float* __restrict_
       }
     }
   } else {
-    for (int sp = 0; sp < splits; ++sp) {
-      const float* pr = ws + sp * stride + (size_t)row * ldp + c0;
+    // Unaligned rows, or a row's last few outputs (columns past the end repeat
+    // the last one and are not stored): single floats, batched alike.
+    constexpr int kBatch = EP::kPair ? 2 : 4;
+    for (int s0 = 0; s0 < splits; s0 += kBatch) {
+      float p[kBatch][8], q[kBatch][8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e)
-        if (c0 + e < ncols) {
-          a[e] += pr[e];
-          if constexpr (EP::kPair) u[e] += pr[ep.width + e];
+      for (int j = 0; j < kBatch; ++j) {
+        const float* pr = ws + (size_t)min(s0 + j, splits - 1) * stride + (size_t)row * ldp;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int c = min(c0 + e, ncols - 1);
+          p[j][e] = pr[c];
+          if constexpr (EP::kPair) q[j][e] = pr[ep.width + c];
         }
+      }
+#pragma unroll
+      for (int j = 0; j < kBatch; ++j) {
+        if (s0 + j >= splits) break;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          a[e] += p[j][e];
+          if constexpr (EP::kPair) u[e] += q[j][e];
+        }
+      }
     }
   }
   uint32_t w[4];
@@ -1065,7 +1081,7 @@ hipError_t tile::launch_sum(const SplitWs& ws, int splits, int m, int ncols, int
   const dim3 grid((unsigned)((threads + 255) / 256));
   // 16-byte partial loads: ws 16-byte aligned and every row / pair offset a
   // multiple of four floats.
-  bool vload = ldp % 4 == 0 && ncols % 8 == 0 && ((uintptr_t)ws.p & 15u) == 0;
+  bool vload = ldp % 4 == 0 && ((uintptr_t)ws.p & 15u) == 0;
   if constexpr (EP::kPair) vload = vload && ep.width % 4 == 0;
   hipLaunchKernelGGL((reduce_ep_kernel<T, EP>), grid, dim3(256), 0, stream, ws.p, splits, m, ncols,
                      ldp, vload, ep);
