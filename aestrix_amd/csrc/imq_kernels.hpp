@@ -54,12 +54,9 @@ hipError_t launch_qgemv_swiglu_norm(const uint32_t* w, const void* scales, const
 // fp32 scratch for split-K partial sums.  With too few output tiles to fill
 // the chip, the MFMA kernel splits K, writes each split's partial sums here
 // and a second kernel adds them; a null or short workspace runs unsplit.
-// cus: the compute units the tile planner counts on (0: the device's); a
-// launch that shares the GPU with another stream's plans for its share.
 struct SplitWs {
   float* p = nullptr;
   size_t bytes = 0;
-  int cus = 0;
 };
 
 // y[m][n] = x . deq(W)^T, any m >= 1, T in {bf16, f16}; MFMA.
@@ -131,6 +128,34 @@ hipError_t launch_qgemm_swiglu(const uint32_t* w, const void* scales, const void
                                const void* x, void* y, int ldy, int k, int n, int m, int width,
                                int gate_row, int up_row, float in_scale, float out_scale, int dtype,
                                hipStream_t stream, SplitWs ws = {});
+
+// Several products of one K and N (a multiple of 256) with one output stage in
+// one launch: the tiles of all share the CUs without a second stream, each
+// row its own product's.  kStore: y (T) [m, n]; kGateAdd: y (fp32) = residual +
+// gate * float(T(acc)), K split where the plan does and ws holds the partial
+// sums (qgemm_group_split_bytes); kSwiGLU: y (T) [m, width] of n = 2 width
+// weight rows, gate rows first.  (Weak, like every launcher that only step.cpp
+// and cond.cpp call: a host-only build of those leaves it out.)
+struct QgemmGroup {
+  enum Stage { kStore, kGateAdd, kSwiGLU };
+  struct Product {
+    const uint32_t* w;
+    const void* scales;
+    const void* biases;
+    const void* x;
+    void* y;
+    const float* residual;
+    const float* gate;
+    int m;
+  };
+  Product p[6];
+  int count;
+  Stage stage;
+  int width;
+};
+__attribute__((weak)) hipError_t launch_qgemm_group(const QgemmGroup& g, int k, int n, int dtype,
+                                                    hipStream_t stream, SplitWs ws = {});
+__attribute__((weak)) size_t qgemm_group_split_bytes(int k, int n, const int* ms, int count);
 
 // y[i] (T) = T(x[i] / scale) for i < count, x fp32; T in {bf16, f16}; with
 // scale_dev the scale is read from device memory when the kernel runs.

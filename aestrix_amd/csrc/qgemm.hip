@@ -30,9 +30,7 @@ namespace {
 // two) against 70.3 (192 x 128 unsplit).  It stays for outputs whose partial
 // sums of even two splits outgrow the static scratch (8.4 M outputs): there
 // both pick alike, and the shapes that the allocation-free entry refuses stay
-// the same; and for launches that share the CUs with another stream's (shared),
-// whose 256-column tiles leave the L2 to both: a denoise step of 1512 + 512
-// rows 1633 us with it, 1661 with kFit.  Below that size a split's partial sums fit that scratch.
+// the same.  Below that size a split's partial sums fit that scratch.
 struct CostModel {
   double step2[9], step1[9];  // per K-step, by mt: 256 and 128 columns
   double round2, round1;      // per round of tiles
@@ -53,11 +51,13 @@ constexpr size_t kLargeMaxPanel = (size_t)4 << 20;  // of a 128-column tile's ac
 // Tile and K split of a launch over n weight rows (split: K may be split;
 // pair: a gate/up pair, whose wave holds gate and up columns: 256-column tiles
 // of 128 rows and more).  Splits are taken only when the tiles leave CUs idle.
-BigPlan pick_big_plan(int m, int n, int k, int cus, bool split, bool pair = false,
-                      bool shared = false) {
+// ms: the rows of each of `count` products of one launch.
+BigPlan pick_big_plan(const int* ms, int count, int n, int k, int cus, bool split, bool pair) {
+  int m = 0;
+  for (int i = 0; i < count; ++i) m += ms[i];
   const int steps = (k + 255) / 256 * 2;  // of 128, whole scale blocks
   const bool tail = k % 256 != 0;
-  const bool large = shared || (size_t)m * n * 8 > kStaticScratchBytes;
+  const bool large = (size_t)m * n * 8 > kStaticScratchBytes;
   const CostModel& c = large ? kLarge : kFit;
   BigPlan best{8, 2, 1, steps};
   double best_cost = 1e30;
@@ -71,7 +71,9 @@ BigPlan pick_big_plan(int m, int n, int k, int cus, bool split, bool pair = fals
       if (nt == 1 && mt == 1) continue;
       // K % 256 != 0 is built for fewer tiles (tile::tile_built).
       if (tail && (nt == 1 ? mt > 4 : mt == 5 || mt == 7)) continue;
-      const long tiles = (long)((m + 32 * mt - 1) / (32 * mt)) * tiles_n;
+      if (count > 1 && !tile::group_built(mt, nt)) continue;
+      long tiles = 0;
+      for (int i = 0; i < count; ++i) tiles += (long)((ms[i] + 32 * mt - 1) / (32 * mt)) * tiles_n;
       // Up to two rounds of workgroups (the former model: any).
       const int max_splits =
           !split || tiles >= cus ? 1
@@ -96,6 +98,10 @@ BigPlan pick_big_plan(int m, int n, int k, int cus, bool split, bool pair = fals
     }
   }
   return best;
+}
+
+BigPlan pick_big_plan(int m, int n, int k, int cus, bool split, bool pair = false) {
+  return pick_big_plan(&m, 1, n, k, cus, split, pair);
 }
 
 // 16-byte alignment of an output or residual pointer (vector output stores).
@@ -151,10 +157,10 @@ hipError_t launch_big_ep(const uint32_t* w, const uint16_t* scales, const uint16
     up_row = ep.up_row;
   }
   const bool tail = k % 256 != 0;
-  const int cus = ws.cus > 0 ? ws.cus : device_cus();
-  BigPlan p = pick_big_plan(m, cols, k, cus, ws.p != nullptr, EP::kPair, ws.cus > 0);
+  const int cus = device_cus();
+  BigPlan p = pick_big_plan(m, cols, k, cus, ws.p != nullptr, EP::kPair);
   if (p.splits > 1 && ws.bytes < (size_t)p.splits * m * cols * sizeof(float))
-    p = pick_big_plan(m, cols, k, cus, false, EP::kPair, ws.cus > 0);  // no room for the partial sums
+    p = pick_big_plan(m, cols, k, cus, false, EP::kPair);  // no room for the partial sums
   if (p.splits == 1)
     return tail ? tile::launch_plan<T, EP, true>(p, w, scales, biases, x, ep, k, n, m, stream)
                 : tile::launch_plan<T, EP, false>(p, w, scales, biases, x, ep, k, n, m, stream);
@@ -326,7 +332,7 @@ hipError_t launch_reduce_swiglu(const float* ws, int splits, int m, int width, v
                                 float in_scale, float out_scale, int dtype, hipStream_t stream) {
   auto* yy = static_cast<uint16_t*>(y);
   const bool vec = al16(y) && ldy % 8 == 0;
-  const SplitWs sw{const_cast<float*>(ws), 0, 0};
+  const SplitWs sw{const_cast<float*>(ws), 0};
   switch (dtype) {
     case kBf16:
       return tile::launch_sum<kBf16>(
@@ -362,6 +368,117 @@ hipError_t launch_qgemm_swiglu(const uint32_t* w, const void* scales, const void
           stream, ws);
     default: return hipErrorInvalidValue;
   }
+}
+
+namespace {
+
+template <int T>
+hipError_t launch_group_t(const QgemmGroup& in, int k, int n, hipStream_t stream, SplitWs ws) {
+  const int cus = device_cus();
+  int ms[tile::kMaxGroup], m = 0;
+  for (int i = 0; i < in.count; ++i) m += ms[i] = in.p[i].m;
+  const bool pair = in.stage == QgemmGroup::kSwiGLU;
+  const int cols = pair ? 2 * in.width : n;
+  auto fill = [&](auto& g) {
+    g.count = in.count;
+    for (int i = 0; i < in.count; ++i) {
+      g.p[i].w = in.p[i].w;
+      g.p[i].scales = static_cast<const uint16_t*>(in.p[i].scales);
+      g.p[i].biases = static_cast<const uint16_t*>(in.p[i].biases);
+      g.p[i].x = static_cast<const uint16_t*>(in.p[i].x);
+      g.p[i].m = in.p[i].m;
+    }
+  };
+  // Only the gated residual adds run with K long enough to split.
+  const bool can_split = in.stage == QgemmGroup::kGateAdd && ws.p != nullptr;
+  BigPlan p = pick_big_plan(ms, in.count, cols, k, cus, can_split, pair);
+  if (p.splits > 1 && ws.bytes < (size_t)p.splits * m * cols * sizeof(float))
+    p = pick_big_plan(ms, in.count, cols, k, cus, false, pair);
+  if (in.stage == QgemmGroup::kStore) {
+    tile::Group<EpStore<T>> g{};
+    fill(g);
+    for (int i = 0; i < in.count; ++i) {
+      auto* y = static_cast<uint16_t*>(in.p[i].y);
+      g.p[i].ep = EpStore<T>{y, n, al16(y) && n % 8 == 0};
+    }
+    return tile::launch_group<T, EpStore<T>>(p, g, k, n, stream);
+  }
+  if (pair) {
+    tile::Group<EpSwiGLU<T>> g{};
+    fill(g);
+    for (int i = 0; i < in.count; ++i) {
+      auto* y = static_cast<uint16_t*>(in.p[i].y);
+      g.p[i].ep = EpSwiGLU<T>{y, in.width, in.width, 0, in.width, 1.0f, 1.0f,
+                              al16(y) && in.width % 8 == 0};
+    }
+    return tile::launch_group<T, EpSwiGLU<T>>(p, g, k, n, stream);
+  }
+  auto ep = [&](int i) {
+    const QgemmGroup::Product& r = in.p[i];
+    auto* y = static_cast<float*>(r.y);
+    const bool vec = al16(y) && al16(r.residual) && al16(r.gate) && n % 4 == 0;
+    return EpGateAdd<T>{y, r.residual, r.gate, n, 1.0f, vec, nullptr};
+  };
+  if (p.splits == 1) {
+    tile::Group<EpGateAdd<T>> g{};
+    fill(g);
+    for (int i = 0; i < in.count; ++i) g.p[i].ep = ep(i);
+    return tile::launch_group<T, EpGateAdd<T>>(p, g, k, n, stream);
+  }
+  // Partial sums of product i after those of the products before it.
+  tile::Group<EpPartial<false>> g{};
+  fill(g);
+  float* part = ws.p;
+  for (int i = 0; i < in.count; ++i) {
+    g.p[i].ep = EpPartial<false>{part, n, n, 0, 0};
+    part += (size_t)p.splits * ms[i] * n;
+  }
+  hipError_t e = tile::launch_group<T, EpPartial<false>>(p, g, k, n, stream);
+  for (int i = 0; i < in.count && e == hipSuccess; ++i)
+    e = tile::launch_sum<T, EpGateAdd<T>>(SplitWs{g.p[i].ep.ws, 0}, p.splits, ms[i], n, n, ep(i),
+                                          stream);
+  return e;
+}
+
+}  // namespace
+
+hipError_t launch_qgemm_group(const QgemmGroup& g, int k, int n, int dtype, hipStream_t stream,
+                              SplitWs ws) {
+  if (g.count < 1 || g.count > tile::kMaxGroup || k % 256 != 0) return hipErrorInvalidValue;
+  bool fits = true;
+  for (int i = 0; i < g.count; ++i) fits = fits && qgemm_big_supported(k, n, g.p[i].m);
+  if (!fits) {  // operands past 32-bit offsets: one after the other
+    hipError_t e = hipSuccess;
+    for (int i = 0; i < g.count && e == hipSuccess; ++i) {
+      const QgemmGroup::Product& p = g.p[i];
+      switch (g.stage) {
+        case QgemmGroup::kStore:
+          e = launch_qgemm(p.w, p.scales, p.biases, p.x, p.y, k, n, p.m, dtype, stream);
+          break;
+        case QgemmGroup::kSwiGLU:
+          e = launch_qgemm_swiglu(p.w, p.scales, p.biases, p.x, p.y, g.width, k, n, p.m, g.width, 0,
+                                  g.width, 1.0f, 1.0f, dtype, stream, SplitWs{});
+          break;
+        default:
+          e = launch_qgemm_gate_add(p.w, p.scales, p.biases, p.x, p.residual, p.gate,
+                                    static_cast<float*>(p.y), k, n, p.m, 1.0f, dtype, stream, ws,
+                                    nullptr);
+      }
+    }
+    return e;
+  }
+  switch (dtype) {
+    case kBf16: return launch_group_t<kBf16>(g, k, n, stream, ws);
+    case kF16: return launch_group_t<kF16>(g, k, n, stream, ws);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+size_t qgemm_group_split_bytes(int k, int n, const int* ms, int count) {
+  int m = 0;
+  for (int i = 0; i < count; ++i) m += ms[i];
+  const BigPlan p = pick_big_plan(ms, count, n, k, device_cus(), true, false);
+  return p.splits > 1 ? (size_t)p.splits * m * n * sizeof(float) : 0;
 }
 
 }  // namespace imq

@@ -31,6 +31,30 @@ template <int T, class EP>
 hipError_t launch_sum(const SplitWs& ws, int splits, int m, int ncols, int ldp, const EP& ep,
                       hipStream_t stream);
 
+// Up to kMaxGroup products of one K, N and output stage for one launch:
+// activations of m rows, and the tiles' ids from `first` on (launch_group
+// fills first and tiles_m).
+constexpr int kMaxGroup = 6;
+template <class EP>
+struct Product {
+  const uint32_t* w;
+  const uint16_t* scales;
+  const uint16_t* biases;
+  const uint16_t* x;
+  EP ep;
+  int m, tiles_m, first;
+};
+template <class EP>
+struct Group {
+  Product<EP> p[kMaxGroup];
+  int count;
+};
+// By plan p: every product's tiles of that size in one grid (K % 256 == 0).
+// Built for 128 rows and more, 128 columns at 128, 192 and 256 rows.
+template <int T, class EP>
+hipError_t launch_group(const BigPlan& p, Group<EP>& g, int k, int n, hipStream_t stream);
+constexpr bool group_built(int mt, int nt) { return mt >= 4 && (nt == 2 || mt % 2 == 0); }
+
 // Tiles built for stage EP (mt: 32-row units, nt: 128-column units).
 template <int T, class EP, bool KT>
 constexpr bool tile_built(int mt, int nt) {

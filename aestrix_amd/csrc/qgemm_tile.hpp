@@ -48,13 +48,13 @@ constexpr int kThreads = 256;
 constexpr int kGroupM = 4;
 constexpr int kXcds = 8;
 
-__device__ __forceinline__ void tile_coords(int bid, int tiles_m, int tiles_n, int& tm, int& tn) {
-  const int total = tiles_m * tiles_n;
-  int id = bid;
-  if (total % kXcds == 0) {
-    const int per = total / kXcds;
-    id = (bid % kXcds) * per + bid / kXcds;
-  }
+// Tile id of workgroup bid of `total`: a contiguous stretch for each XCD.
+__device__ __forceinline__ int xcd_order(int bid, int total) {
+  return total % kXcds == 0 ? (bid % kXcds) * (total / kXcds) + bid / kXcds : bid;
+}
+
+// Tile id's place in the raster.
+__device__ __forceinline__ void raster(int id, int tiles_m, int tiles_n, int& tm, int& tn) {
   const int per_group = kGroupM * tiles_n;
   const int grp = id / per_group;
   const int first_m = grp * kGroupM;
@@ -62,6 +62,10 @@ __device__ __forceinline__ void tile_coords(int bid, int tiles_m, int tiles_n, i
   const int in = id - grp * per_group;
   tm = first_m + in % gsz;
   tn = in / gsz;
+}
+
+__device__ __forceinline__ void tile_coords(int bid, int tiles_m, int tiles_n, int& tm, int& tn) {
+  raster(xcd_order(bid, tiles_m * tiles_n), tiles_m, tiles_n, tm, tn);
 }
 
 // LDS slot of 16-byte chunk c (0..7) of activation-tile row r.  Conflict-free
@@ -773,10 +777,11 @@ __device__ __forceinline__ void big_write_tile(const EP& ep, const BigRing& ring
 // a taller tile (each dequantized weight fragment feeds MT MFMAs; at one or
 // two row tiles the dequant VALU work, not the matrix core, bounds a step).
 template <int T, int MT, int NT, class EP, bool KT>
-__global__ __launch_bounds__(kThreads, 1) void qgemm_big_kernel(
-    const uint32_t* __restrict__ w, const uint16_t* __restrict__ scales,
-    const uint16_t* __restrict__ biases, const uint16_t* __restrict__ x, const EP ep,
-    int M, int N, int K, int tiles_m, int tiles_n, int split_steps) {
+__device__ __forceinline__ void big_tile(const uint32_t* __restrict__ w,
+                                         const uint16_t* __restrict__ scales,
+                                         const uint16_t* __restrict__ biases,
+                                         const uint16_t* __restrict__ x, const EP& ep, int M, int N,
+                                         int K, int tm, int tn, int split_steps) {
   static_assert(NT == 1 || NT == 2, "one or two 32-column tiles per wave");
   static_assert(!EP::kPair || NT == 2, "a gate/up pair takes two column tiles per wave");
   using C = BigCfg<MT>;
@@ -789,8 +794,6 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_big_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r32 = lane & 31;
   const int h = lane >> 5;
-  int tm, tn;
-  tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
   const int m0 = tm * C::kBM;
   const int n0 = tn * (128 * NT);
   const int arow0 = 0;                      // every wave covers all rows of the tile
@@ -963,6 +966,16 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_big_kernel(
 }
 
 template <int T, int MT, int NT, class EP, bool KT>
+__global__ __launch_bounds__(kThreads, 1) void qgemm_big_kernel(
+    const uint32_t* __restrict__ w, const uint16_t* __restrict__ scales,
+    const uint16_t* __restrict__ biases, const uint16_t* __restrict__ x, const EP ep,
+    int M, int N, int K, int tiles_m, int tiles_n, int split_steps) {
+  int tm, tn;
+  tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  big_tile<T, MT, NT, EP, KT>(w, scales, biases, x, ep, M, N, K, tm, tn, split_steps);
+}
+
+template <int T, int MT, int NT, class EP, bool KT>
 hipError_t launch_big(const BigPlan& p, const uint32_t* w, const uint16_t* scales,
                       const uint16_t* biases, const uint16_t* x, const EP& ep, int k, int n, int m,
                       hipStream_t stream) {
@@ -1072,6 +1085,24 @@ __global__ __launch_bounds__(256) void reduce_ep_kernel(const float* __restrict_
   }
 }
 
+// Several products of one K, N and output stage in one launch, the tiles of all
+// in one grid (tile::Group).
+template <int T, int MT, int NT, class EP>
+__global__ __launch_bounds__(kThreads, 1) void qgemm_big_kernel(const tile::Group<EP> g, int N,
+                                                                     int K, int tiles_n,
+                                                                     int split_steps) {
+  const int id = xcd_order(blockIdx.x, (int)gridDim.x);
+  // The product this tile belongs to, by compares and selects (the argument
+  // block indexed by a variable would be copied to scratch memory).
+  tile::Product<EP> p = g.p[0];
+#pragma unroll
+  for (int i = 1; i < tile::kMaxGroup; ++i)
+    if (i < g.count && id >= g.p[i].first) p = g.p[i];
+  int tm, tn;
+  raster(id - p.first, p.tiles_m, tiles_n, tm, tn);
+  big_tile<T, MT, NT, EP, false>(p.w, p.scales, p.biases, p.x, p.ep, p.m, N, K, tm, tn, split_steps);
+}
+
 }  // namespace
 
 template <int T, class EP>
@@ -1130,6 +1161,40 @@ hipError_t tile::launch_plan(const BigPlan& p, const uint32_t* w, const uint16_t
 #undef IMQ_TILE
 }
 
+template <int T, class EP>
+hipError_t tile::launch_group(const BigPlan& p, Group<EP>& g, int k, int n, hipStream_t stream) {
+  int cols = n;
+  if constexpr (EP::kPair) cols = 2 * g.p[0].ep.width;
+  const int tiles_n = (cols + 128 * p.nt - 1) / (128 * p.nt);
+  int tiles = 0;
+  for (int i = 0; i < g.count; ++i) {
+    g.p[i].first = tiles;
+    g.p[i].tiles_m = (g.p[i].m + 32 * p.mt - 1) / (32 * p.mt);
+    tiles += g.p[i].tiles_m * tiles_n;
+  }
+  const dim3 grid((unsigned)tiles, (unsigned)p.splits);
+#define IMQ_TILE(MT, NT)                                                                         \
+  case 10 * MT + NT:                                                                             \
+    if constexpr (tile::tile_built<T, EP, false>(MT, NT)) {                                      \
+      hipLaunchKernelGGL((qgemm_big_kernel<T, MT, NT, EP>), grid, dim3(kThreads), 0, stream,    \
+                         g, n, k, tiles_n, p.split_steps);                                       \
+      return hipGetLastError();                                                                  \
+    }                                                                                            \
+    return hipErrorInvalidValue
+  switch (10 * p.mt + p.nt) {
+    IMQ_TILE(4, 2);
+    IMQ_TILE(5, 2);
+    IMQ_TILE(6, 2);
+    IMQ_TILE(7, 2);
+    IMQ_TILE(8, 2);
+    IMQ_TILE(4, 1);
+    IMQ_TILE(6, 1);
+    IMQ_TILE(8, 1);
+    default: return hipErrorInvalidValue;
+  }
+#undef IMQ_TILE
+}
+
 // Every launch of one output stage (fused and plain) for element type T.
 #define IMQ_TILE_STAGE(T, ...)                                                                     \
   template hipError_t tile::launch_reg<T, __VA_ARGS__>(                                            \
@@ -1149,6 +1214,9 @@ hipError_t tile::launch_plan(const BigPlan& p, const uint32_t* w, const uint16_t
   IMQ_TILE_PLAN(T, KT, EpSwiGLU<T>);        \
   IMQ_TILE_PLAN(T, KT, EpPartial<false>);   \
   IMQ_TILE_PLAN(T, KT, EpPartial<true>)
+#define IMQ_TILE_GROUP(T, ...)                                                                   \
+  template hipError_t tile::launch_group<T, __VA_ARGS__>(const BigPlan&, Group<__VA_ARGS__>&, int, \
+                                                         int, hipStream_t)
 #define IMQ_TILE_STAGES(T)            \
   IMQ_TILE_STAGE(T, EpStore<T>);      \
   IMQ_TILE_STAGE(T, EpResidAdd<T>);   \

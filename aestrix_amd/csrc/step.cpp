@@ -39,16 +39,7 @@ struct imq_dit_step {
   float* norm_w = nullptr;  // fp32 [dim]
   float* gates = nullptr;   // fp32 [4 n_double + n_single][dim]
   imq::SplitWs split;       // partial sums of the projections that split K
-  imq::SplitWs split_txt;   // the same for the double blocks' text rows (side stream)
-  // CUs the double blocks' image / text chains plan for where they run side by
-  // side (rows in proportion, the text share rounded up).
-  int cus_img = 0, cus_txt = 0;
   hipStream_t cap = nullptr;
-  // The double blocks' text-row projections run on `side`, beside the image
-  // rows on the main stream, forked and joined by these events.
-  hipStream_t side = nullptr;
-  hipEvent_t ev_fork = nullptr;
-  hipEvent_t ev_join = nullptr;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   int launches = 0;
@@ -76,42 +67,27 @@ constexpr float kEps = 1e-5f;  // DirectDiTStep.swift:416
 
 size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 
-// The block halves share this launch bookkeeping: every kernel launched
-// counts in st->launches, the first failing call's error is kept, and the
-// text rows' chain (on st->side) forks from and joins back into stream s.
+// The block halves share this launch bookkeeping: every norm, product and
+// scaling counts in st->launches (a grouped launch as many as it holds), and
+// the first failing call's error is kept.
 struct Enc {
   imq_dit_step* st;
   hipStream_t s;
   hipError_t e = hipSuccess;
-  void ok(hipError_t r) {
-    ++st->launches;
+  void ok(hipError_t r, int count = 1) {
+    st->launches += count;
     if (e == hipSuccess) e = r;
   }
   void sync(hipError_t r) {
     if (e == hipSuccess) e = r;
   }
-  void fork() {
-    sync(hipEventRecord(st->ev_fork, s));
-    sync(hipStreamWaitEvent(st->side, st->ev_fork, 0));
+  // A product of the launch g (gate: the residual add's, into y).
+  static void add(imq::QgemmGroup& g, const imq_qweight& w, const void* x, void* y, int m,
+                  const float* gate = nullptr) {
+    g.p[g.count++] = {w.w, w.scales, w.biases, x, y, static_cast<const float*>(y), gate, m};
   }
-  void join() {
-    sync(hipEventRecord(st->ev_join, st->side));
-    sync(hipStreamWaitEvent(s, st->ev_join, 0));
-  }
-  // The image and text chains each plan their tiles for their share of the
-  // CUs, so that both fit side by side in one tile round: at 4096 + 512 rows
-  // and dim 3072, 192 + 24 tiles of 256 rows on 256 CUs instead of the 228
-  // tiles of 224 rows the image rows take alone.  The SwiGLU projections keep
-  // the whole device (1152 tiles, 4.5 rounds): the text rows fill the last.
-  imq::SplitWs wi() const {
-    imq::SplitWs w = st->split;
-    w.cus = st->cus_img;
-    return w;
-  }
-  imq::SplitWs wt() const {
-    imq::SplitWs w = st->split_txt;
-    w.cus = st->cus_txt;
-    return w;
+  void group(const imq::QgemmGroup& g, int k, int n) {
+    ok(imq::launch_qgemm_group(g, k, n, (int)st->dtype, s, st->split), g.count);
   }
   static const char* rows(const void* base, int row0, int width) {
     return static_cast<const char*>(base) + (size_t)row0 * width * 2;
@@ -133,25 +109,24 @@ struct Enc {
 // Double block b before attention (encodeDouble's projections up to the
 // attention, DirectDiTStep.swift:549-563): q, k, v of the text rows (add_q,
 // add_k, add_v) and of the image rows (to_q, to_k, to_v) from the normalized
-// input.  Image rows (4096 at 1024^2) on s and text rows (512) on the side
-// stream at the same time: an image-row projection leaves CUs idle in its
-// last tile round and a text-row one never fills the GPU.  The two chains
-// touch disjoint rows of every buffer and have their own split-K workspaces.
+// input, all six in one launch: the tiles of an image-row product leave CUs
+// idle in their last round and a text-row one never fills the GPU, alone.  The
+// whole double block at 1024 + 512 rows (dim 3072, f16) took 543 us as two
+// chains on two streams, each planned for its share of the CUs, and 399 us as
+// grouped launches; 799 + 512 rows (1536) 199 / 121; level at 4096 + 512 rows.
 void double_attn_in(Enc& c, int b, const float* x, const void* nx, void* q, void* k, void* v) {
   imq_dit_step* st = c.st;
   const imq_dit_dims& d = st->d;
-  const int dim = d.dim, T = (int)st->dtype;
+  const int dim = d.dim;
   const imq_qweight* W = &st->w[(size_t)12 * b];
   const void* n = c.norm(x, nx);
   void* outs[3] = {q, k, v};
-  c.fork();
+  imq::QgemmGroup g{};
+  g.stage = imq::QgemmGroup::kStore;
   for (int i = 0; i < 3; ++i)
-    c.ok(imq::launch_qgemm(W[i].w, W[i].scales, W[i].biases, Enc::rows(n, d.l_txt, dim),
-                           Enc::rows(outs[i], d.l_txt, dim), dim, dim, d.l_img, T, c.s, c.wi()));
-  for (int i = 0; i < 3; ++i)
-    c.ok(imq::launch_qgemm(W[3 + i].w, W[3 + i].scales, W[3 + i].biases, n, outs[i], dim, dim,
-                           d.l_txt, T, st->side, c.wt()));
-  c.join();
+    c.add(g, W[i], Enc::rows(n, d.l_txt, dim), Enc::rows(outs[i], d.l_txt, dim), d.l_img);
+  for (int i = 0; i < 3; ++i) c.add(g, W[3 + i], n, outs[i], d.l_txt);
+  c.group(g, dim, dim);
 }
 
 // Double block b after attention (:568-571): the image rows' to_out and the
@@ -160,50 +135,48 @@ void double_attn_in(Enc& c, int b, const float* x, const void* nx, void* q, void
 void double_attn_out(Enc& c, int b, const void* attn, float* x) {
   imq_dit_step* st = c.st;
   const imq_dit_dims& d = st->d;
-  const int dim = d.dim, T = (int)st->dtype;
+  const int dim = d.dim;
   const imq_qweight* W = &st->w[(size_t)12 * b];
-  const float* g = st->gates + (size_t)4 * b * dim;
-  float* Xt = x;
-  float* Xi = x + (size_t)d.l_txt * dim;
-  c.fork();
-  c.ok(imq::launch_qgemm_gate_add(W[6].w, W[6].scales, W[6].biases, Enc::rows(attn, d.l_txt, dim),
-                                  Xi, g, Xi, dim, dim, d.l_img, 1.0f, T, c.s, c.wi()));
-  c.ok(imq::launch_qgemm_gate_add(W[7].w, W[7].scales, W[7].biases, attn, Xt, g + dim, Xt, dim,
-                                  dim, d.l_txt, 1.0f, T, st->side, c.wt()));
-  c.join();
+  const float* gates = st->gates + (size_t)4 * b * dim;
+  imq::QgemmGroup g{};
+  g.stage = imq::QgemmGroup::kGateAdd;
+  c.add(g, W[6], Enc::rows(attn, d.l_txt, dim), x + (size_t)d.l_txt * dim, d.l_img, gates);
+  c.add(g, W[7], attn, x, d.l_txt, gates + dim);
+  c.group(g, dim, dim);
 }
 
 // Double block b's MLPs (:572-587): SwiGLU(nx . linear_in^T) then
 // linear_out with the gated residual add, image rows (ff) and text rows
-// (ff_context) side by side.
+// (ff_context) in one launch each.
 void double_mlp(Enc& c, int b, const void* nx, float* x) {
   imq_dit_step* st = c.st;
   const imq_dit_dims& d = st->d;
-  const int dim = d.dim, ffi = d.ff_inner, T = (int)st->dtype;
+  const int dim = d.dim, ffi = d.ff_inner;
   const imq_qweight* W = &st->w[(size_t)12 * b];
-  const float* g = st->gates + (size_t)4 * b * dim;
-  float* Xt = x;
-  float* Xi = x + (size_t)d.l_txt * dim;
+  const float* gates = st->gates + (size_t)4 * b * dim;
   const void* n = c.norm(x, nx);
-  c.fork();
-  c.ok(imq::launch_qgemm_swiglu(W[8].w, W[8].scales, W[8].biases, Enc::rows(n, d.l_txt, dim),
-                                Enc::rows(st->SW, d.l_txt, ffi), ffi, dim, 2 * ffi, d.l_img, ffi, 0,
-                                ffi, 1.0f, 1.0f, T, c.s, st->split));
-  c.ok(imq::launch_qgemm_gate_add(W[9].w, W[9].scales, W[9].biases,
-                                  Enc::rows(st->SW, d.l_txt, ffi), Xi, g + 2 * dim, Xi, ffi, dim,
-                                  d.l_img, 1.0f, T, c.s, c.wi()));
-  c.ok(imq::launch_qgemm_swiglu(W[10].w, W[10].scales, W[10].biases, n, st->SW, ffi, dim, 2 * ffi,
-                                d.l_txt, ffi, 0, ffi, 1.0f, 1.0f, T, st->side, st->split_txt));
-  c.ok(imq::launch_qgemm_gate_add(W[11].w, W[11].scales, W[11].biases, st->SW, Xt, g + 3 * dim, Xt,
-                                  ffi, dim, d.l_txt, 1.0f, T, st->side, c.wt()));
-  c.join();
+  imq::QgemmGroup in{};
+  in.stage = imq::QgemmGroup::kSwiGLU;
+  in.width = ffi;
+  c.add(in, W[8], Enc::rows(n, d.l_txt, dim), Enc::rows(st->SW, d.l_txt, ffi), d.l_img);
+  c.add(in, W[10], n, st->SW, d.l_txt);
+  c.group(in, dim, 2 * ffi);
+  imq::QgemmGroup out{};
+  out.stage = imq::QgemmGroup::kGateAdd;
+  c.add(out, W[9], Enc::rows(st->SW, d.l_txt, ffi), x + (size_t)d.l_txt * dim, d.l_img,
+        gates + 2 * dim);
+  c.add(out, W[11], st->SW, x, d.l_txt, gates + 3 * dim);
+  c.group(out, ffi, dim);
 }
 
 // Single block b before attention (encodeSingle up to the attention,
 // :593-611): the Q/K/V rows of to_qkv_mlp_proj into qkv and its SwiGLU rows
-// into columns [dim, dim + ff_inner) of concat.  Both read the same input and
-// write different buffers, so they run side by side (Q/K/V on the side
-// stream): each one's part-empty last tile round fills with the other's tiles.
+// into columns [dim, dim + ff_inner) of concat, one after the other.  Side by
+// side on two streams each would fill the other's part-empty last round, but
+// the fork and join cost more at every size: single block of 300 + 60 rows
+// (dim 1536) 59.3 against 50.9 us, 828 + 60 (2048) 133 / 120, 1024 + 512
+// (3072) 376 / 366, 4096 + 512 1007 / 1002; a step graph of 2 double and 8
+// single blocks 3778 / 3724 us at 1024 + 512 rows, 10048 / 10021 at 4096 + 512.
 void single_attn_in(Enc& c, int b, const float* x, const void* nx, void* qkv, void* concat) {
   imq_dit_step* st = c.st;
   const imq_dit_dims& d = st->d;
@@ -211,14 +184,12 @@ void single_attn_in(Enc& c, int b, const float* x, const void* nx, void* qkv, vo
   const int cw = dim + ffi;
   const imq_qweight* W = &st->w[(size_t)12 * d.n_double + 2 * b];
   const void* n = c.norm(x, nx);
-  c.fork();
-  c.ok(imq::launch_qgemm(W[0].w, W[0].scales, W[0].biases, n, qkv, dim, 3 * dim, J, T, st->side,
-                         st->split_txt));
+  c.ok(imq::launch_qgemm(W[0].w, W[0].scales, W[0].biases, n, qkv, dim, 3 * dim, J, T, c.s,
+                         st->split));
   c.ok(imq::launch_qgemm_swiglu(W[0].w, W[0].scales, W[0].biases, n,
                                 static_cast<char*>(concat) + (size_t)dim * 2, cw, dim,
                                 3 * dim + 2 * ffi, J, ffi, 3 * dim, 3 * dim + ffi, 1.0f, 1.0f, T,
                                 c.s, st->split));
-  c.join();
 }
 
 // Single block b after attention (:616-617): to_out over [attention | MLP]
@@ -308,9 +279,6 @@ void release(imq_dit_step* st) {
   if (st->exec) (void)hipGraphExecDestroy(st->exec);
   if (st->graph) (void)hipGraphDestroy(st->graph);
   if (st->cap) (void)hipStreamDestroy(st->cap);
-  if (st->side) (void)hipStreamDestroy(st->side);
-  if (st->ev_fork) (void)hipEventDestroy(st->ev_fork);
-  if (st->ev_join) (void)hipEventDestroy(st->ev_join);
   if (st->arena) (void)hipFree(st->arena);
 }
 
@@ -318,13 +286,9 @@ void release(imq_dit_step* st) {
 // (fused ones over their weight rows, 2 * ff_inner for a SwiGLU pair).
 size_t split_bytes(const imq_dit_dims& d) {
   const int J = d.l_txt + d.l_img, ffi = d.ff_inner, cw = d.dim + d.ff_inner;
-  size_t b = 0;
-  for (int m : {d.l_img, d.l_txt}) {
-    b = std::max({b, imq::qgemm_split_bytes(d.dim, d.dim, m),
-                  imq::qgemm_split_bytes(d.dim, d.dim, m, true),
-                  imq::qgemm_split_bytes(d.dim, 2 * ffi, m, true),
-                  imq::qgemm_split_bytes(ffi, d.dim, m, true)});
-  }
+  const int ms[2] = {d.l_img, d.l_txt};
+  const size_t b = std::max(imq::qgemm_group_split_bytes(d.dim, d.dim, ms, 2),
+                            imq::qgemm_group_split_bytes(ffi, d.dim, ms, 2));
   return std::max({b, imq::qgemm_split_bytes(d.dim, 3 * d.dim, J),
                    imq::qgemm_split_bytes(d.dim, 2 * ffi, J, true),
                    imq::qgemm_split_bytes(cw, d.dim, J, true)});
@@ -420,10 +384,9 @@ int imq_dit_step_create(imq_ctx* ctx, const imq_dit_dims* dims, const imq_qweigh
                           J * (d.dim + d.ff_inner) * es,
                           (size_t)d.dim * 4,
                           ((size_t)4 * d.n_double + d.n_single) * d.dim * 4,
-                          split_bytes(d),
                           split_bytes(d)};
-  size_t off[12], total = 0;
-  for (int i = 0; i < 12; ++i) {
+  size_t off[11], total = 0;
+  for (int i = 0; i < 11; ++i) {
     off[i] = total;
     total += align256(sizes[i]);
   }
@@ -448,16 +411,6 @@ int imq_dit_step_create(imq_ctx* ctx, const imq_dit_dims* dims, const imq_qweigh
   st->norm_w = reinterpret_cast<float*>(a + off[8]);
   st->gates = reinterpret_cast<float*>(a + off[9]);
   st->split = imq::SplitWs{reinterpret_cast<float*>(a + off[10]), sizes[10]};
-  st->split_txt = imq::SplitWs{reinterpret_cast<float*>(a + off[11]), sizes[11]};
-  {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        cus <= 0)
-      cus = 256;
-    st->cus_txt = std::max(1, (int)(((size_t)cus * d.l_txt + J - 1) / J));
-    st->cus_img = std::max(1, cus - st->cus_txt);
-  }
   // Zero everything (the attention half of C stays zero), ones for the
   // conditioning vectors.  Plain (uncaptured) memsets at set-up.
   e = hipMemset(st->arena, 0, total);
@@ -465,9 +418,6 @@ int imq_dit_step_create(imq_ctx* ctx, const imq_dit_dims* dims, const imq_qweigh
   if (e == hipSuccess)
     e = hipMemsetD32(st->gates, 0x3F800000u, ((size_t)4 * d.n_double + d.n_single) * d.dim);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&st->cap, hipStreamNonBlocking);
-  if (e == hipSuccess) e = hipStreamCreateWithFlags(&st->side, hipStreamNonBlocking);
-  if (e == hipSuccess) e = hipEventCreateWithFlags(&st->ev_fork, hipEventDisableTiming);
-  if (e == hipSuccess) e = hipEventCreateWithFlags(&st->ev_join, hipEventDisableTiming);
   if (e == hipSuccess) e = hipDeviceSynchronize();
   if (e != hipSuccess) {
     release(st);
