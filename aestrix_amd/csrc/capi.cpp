@@ -440,10 +440,9 @@ int imq_memcpy_d2d(imq_ctx* ctx, void* dst, const void* src, size_t bytes, imq_s
   return copy(ctx, "imq_memcpy_d2d", dst, src, bytes, hipMemcpyDeviceToDevice, stream);
 }
 
-int imq_dequantize_rows(imq_ctx* ctx, const uint32_t* w, const void* scales, const void* biases,
-                        const int32_t* rows, int count, void* out, int k, int n, int group_size,
-                        int bits, imq_dtype dtype, imq_stream stream) {
-  const char* fn = "imq_dequantize_rows";
+static int check_rows(imq_ctx* ctx, const char* fn, const uint32_t* w, const void* scales,
+                      const void* biases, const void* rows, size_t id_bytes, int count,
+                      const void* out, int k, int n, int group_size, int bits, imq_dtype dtype) {
   if (!ctx) return fail(nullptr, IMQ_EINVAL, "%s: null context", fn);
   if (group_size != 64)
     return fail(ctx, IMQ_EUNSUPPORTED, "%s: group_size %d (only 64 is provided)", fn, group_size);
@@ -460,16 +459,41 @@ int imq_dequantize_rows(imq_ctx* ctx, const uint32_t* w, const void* scales, con
                 count, k);
   if (count == 0) return IMQ_OK;
   if (!w || !scales || !biases || !rows || !out)
-    return fail(ctx, IMQ_EINVAL, "%s: null device pointer", fn);
+    return fail(ctx, IMQ_EINVAL, "%s: null pointer", fn);
   const size_t es = elem_size(dtype);
-  if (!aligned(w, 4) || !aligned(rows, 4) || !aligned(out, 16) || !aligned(scales, es) ||
+  if (!aligned(w, 4) || !aligned(rows, id_bytes) || !aligned(out, 16) || !aligned(scales, es) ||
       !aligned(biases, es))
-    return fail(ctx, IMQ_EINVAL, "%s: misaligned pointer (w, rows 4; out 16; scales, biases %zu)",
-                fn, es);
-  int rc = bind_device(ctx);
-  if (rc != IMQ_OK) return rc;
+    return fail(ctx, IMQ_EINVAL,
+                "%s: misaligned pointer (w 4; rows %zu; out 16; scales, biases %zu)", fn, id_bytes,
+                es);
+  return IMQ_OK;
+}
+
+int imq_dequantize_rows(imq_ctx* ctx, const uint32_t* w, const void* scales, const void* biases,
+                        const int32_t* rows, int count, void* out, int k, int n, int group_size,
+                        int bits, imq_dtype dtype, imq_stream stream) {
+  const char* fn = "imq_dequantize_rows";
+  int rc = check_rows(ctx, fn, w, scales, biases, rows, 4, count, out, k, n, group_size, bits, dtype);
+  if (rc != IMQ_OK || count == 0) return rc;
+  if ((rc = bind_device(ctx)) != IMQ_OK) return rc;
   const hipError_t e = imq::launch_dequant_rows(w, scales, biases, rows, count, out, k, n,
                                                 (int)dtype, static_cast<hipStream_t>(stream));
+  return e == hipSuccess ? IMQ_OK : hip_fail(ctx, e, fn);
+}
+
+int imq_dequantize_rows_host(imq_ctx* ctx, const uint32_t* w, const void* scales,
+                             const void* biases, const int64_t* rows, int count, void* out, int k,
+                             int n, int group_size, int bits, imq_dtype dtype, imq_stream stream) {
+  const char* fn = "imq_dequantize_rows_host";
+  int rc = check_rows(ctx, fn, w, scales, biases, rows, 8, count, out, k, n, group_size, bits, dtype);
+  if (rc != IMQ_OK || count == 0) return rc;
+  for (int i = 0; i < count; ++i)
+    if (rows[i] < 0 || rows[i] >= n)
+      return fail(ctx, IMQ_EINVAL, "%s: ids must lie in [0, %d), got %lld at %d", fn, n,
+                  (long long)rows[i], i);
+  if ((rc = bind_device(ctx)) != IMQ_OK) return rc;
+  const hipError_t e = imq::launch_dequant_rows_host(w, scales, biases, rows, count, out, k, n,
+                                                     (int)dtype, static_cast<hipStream_t>(stream));
   return e == hipSuccess ? IMQ_OK : hip_fail(ctx, e, fn);
 }
 

@@ -15,6 +15,9 @@
 // equals the integer formula of DirectTEEncoder.swift:39-43 for every non-NaN
 // value; a NaN result (possible only when a scale or bias is itself inf or
 // NaN) stays a quiet NaN.
+#include <algorithm>
+#include <type_traits>
+
 #include "imq_device.hpp"
 #include "imq_kernels.hpp"
 
@@ -24,6 +27,8 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kWordsPerThread = 4;
 constexpr int kWordsPerBlock = kThreads * kWordsPerThread;
+// Ids a launch of the rows form takes as arguments (3 KiB; a launch takes 4).
+constexpr int kArgRows = 768;
 
 struct Bf16Out {
   using S = uint16_t;
@@ -114,24 +119,39 @@ __global__ __launch_bounds__(kThreads) void dequant_kernel(const uint32_t* __res
 // 1 KiB contiguous; a group's 16-byte piece i sits in slot i ^ (group % 8) of
 // its row, so neither the writes (16 lanes: 16 rows, one piece each) nor the
 // reads (16 lanes: two rows) meet in a bank.  Groups past the end load a
-// clamped duplicate and store nothing.  GATHER: output group g is group
-// g % gpr of W's row rows[g / gpr] (the rows form below), the id clamped to
-// [0, n) so that a bad id never reads outside W.
+// clamped duplicate and store nothing.  With a row source (Rows, below) output
+// group g is group g % gpr of W's row rows(g / gpr), the id clamped to [0, n)
+// so that a bad id never reads outside W.
 constexpr int kStageRow = 8;  // 16-byte LDS slots per group
 
-template <typename Out, bool GATHER = false>
+// Where the rows form takes its ids from: device memory, or the kernel's own
+// argument block.  A prompt's ids start on the host, and at a few dozen rows
+// the copy that brings them to the device took four times as long as the whole
+// kernel (30 rows of 2560: 32.4 us a call with the copy, 9.3 us with the ids
+// as arguments).
+struct AllRows {};
+struct DeviceRows {
+  const int32_t* ids;
+  __device__ __forceinline__ int operator()(uint32_t r) const { return ids[r]; }
+};
+struct ArgRows {
+  int32_t ids[kArgRows];
+  __device__ __forceinline__ int operator()(uint32_t r) const { return ids[r]; }
+};
+
+template <typename Out, typename Rows = AllRows>
 __global__ __launch_bounds__(kThreads) void dequant_group_kernel(
     const uint32_t* __restrict__ w, const typename Out::S* __restrict__ scales,
     const typename Out::S* __restrict__ biases, u32x4_t* __restrict__ out, uint32_t groups,
-    const int32_t* __restrict__ rows = nullptr, uint32_t gpr = 0, int n = 0) {
+    const Rows rows, uint32_t gpr, int n) {
   static_assert(Out::kWordBytes == 16, "16-bit outputs");
   __shared__ u32x4_t stage[kThreads * kStageRow];
   const uint32_t g0 = blockIdx.x * (uint32_t)kThreads;
   const uint32_t go = min(g0 + threadIdx.x, groups - 1);
   size_t g = go;  // the source group
-  if constexpr (GATHER) {
+  if constexpr (!std::is_same<Rows, AllRows>::value) {
     const uint32_t r = go / gpr;
-    const int id = min(max(rows[r], 0), n - 1);
+    const int id = min(max(rows(r), 0), n - 1);
     g = (size_t)id * gpr + (go - r * gpr);
   }
   const u32x4_t* wp = reinterpret_cast<const u32x4_t*>(w) + 2 * g;
@@ -171,15 +191,15 @@ __global__ __launch_bounds__(kThreads) void dequant_group_kernel(
 // Rows gathered by index (DirectTEEncoder.embedRow, :106-123, for a batch of
 // token ids): output row r is deq(W[rows[r]]); ids are clamped to [0, n) so a
 // bad id never reads outside W.  One thread per packed word, as above.
-template <typename Out>
+template <typename Out, typename Rows>
 __global__ __launch_bounds__(kThreads) void dequant_rows_kernel(
     const uint32_t* __restrict__ w, const typename Out::S* __restrict__ scales,
-    const typename Out::S* __restrict__ biases, const int32_t* __restrict__ rows,
-    u32x4_t* __restrict__ out, uint32_t total_words, uint32_t wpr, int n) {
+    const typename Out::S* __restrict__ biases, const Rows rows, u32x4_t* __restrict__ out,
+    uint32_t total_words, uint32_t wpr, int n) {
   const uint32_t o = blockIdx.x * (uint32_t)kThreads + threadIdx.x;
   if (o >= total_words) return;
   const uint32_t r = o / wpr, j = o - r * wpr;
-  const int id = min(max(rows[r], 0), n - 1);
+  const int id = min(max(rows(r), 0), n - 1);
   const size_t wi = (size_t)id * wpr + j;
   const uint32_t word = __builtin_nontemporal_load(w + wi);
   const float s = Out::load(scales[wi >> 3]);
@@ -205,9 +225,9 @@ __global__ __launch_bounds__(kThreads) void dequant_rows_kernel(
   }
 }
 
-template <typename Out>
+template <typename Out, typename Rows>
 hipError_t launch_rows_out(const uint32_t* w, const void* scales, const void* biases,
-                           const int32_t* rows, int count, void* out, int k, int n,
+                           const Rows& rows, int count, void* out, int k, int n,
                            hipStream_t stream) {
   using S = typename Out::S;
   const uint32_t wpr = (uint32_t)(k / 8), total = (uint32_t)count * wpr;
@@ -216,14 +236,14 @@ hipError_t launch_rows_out(const uint32_t* w, const void* scales, const void* bi
   if constexpr (Out::kWordBytes == 16) {
     if (((uintptr_t)w & 15u) == 0) {
       const uint32_t gpr = wpr / 8, groups = (uint32_t)count * gpr;  // K % 64 == 0
-      hipLaunchKernelGGL((dequant_group_kernel<Out, true>),
+      hipLaunchKernelGGL((dequant_group_kernel<Out, Rows>),
                          dim3((groups + kThreads - 1) / kThreads), dim3(kThreads), 0, stream, w,
                          static_cast<const S*>(scales), static_cast<const S*>(biases),
                          static_cast<u32x4_t*>(out), groups, rows, gpr, n);
       return hipGetLastError();
     }
   }
-  hipLaunchKernelGGL(dequant_rows_kernel<Out>, dim3((total + kThreads - 1) / kThreads),
+  hipLaunchKernelGGL((dequant_rows_kernel<Out, Rows>), dim3((total + kThreads - 1) / kThreads),
                      dim3(kThreads), 0, stream, w, static_cast<const S*>(scales),
                      static_cast<const S*>(biases), rows, static_cast<u32x4_t*>(out), total, wpr, n);
   return hipGetLastError();
@@ -244,7 +264,7 @@ hipError_t launch_out(const uint32_t* w, const void* scales, const void* biases,
       hipLaunchKernelGGL(dequant_group_kernel<Out>, dim3((groups + kThreads - 1) / kThreads),
                          dim3(kThreads), 0, stream, w + w0,
                          static_cast<const S*>(scales) + w0 / 8,
-                         static_cast<const S*>(biases) + w0 / 8, op, groups);
+                         static_cast<const S*>(biases) + w0 / 8, op, groups, AllRows{}, 0u, 0);
     } else {
       hipLaunchKernelGGL(dequant_kernel<Out>, grid, dim3(kThreads), 0, stream, w + w0,
                          static_cast<const S*>(scales) + w0 / 8,
@@ -262,12 +282,33 @@ hipError_t launch_dequant_rows(const uint32_t* w, const void* scales, const void
                                const int32_t* rows, int count, void* out, int k, int n, int dtype,
                                hipStream_t stream) {
   if (count <= 0) return hipSuccess;
+  const DeviceRows src{rows};
   switch (dtype) {
-    case kBf16: return launch_rows_out<Bf16Out>(w, scales, biases, rows, count, out, k, n, stream);
-    case kF16: return launch_rows_out<F16Out>(w, scales, biases, rows, count, out, k, n, stream);
-    case kF32: return launch_rows_out<F32Out>(w, scales, biases, rows, count, out, k, n, stream);
+    case kBf16: return launch_rows_out<Bf16Out>(w, scales, biases, src, count, out, k, n, stream);
+    case kF16: return launch_rows_out<F16Out>(w, scales, biases, src, count, out, k, n, stream);
+    case kF32: return launch_rows_out<F32Out>(w, scales, biases, src, count, out, k, n, stream);
     default: return hipErrorInvalidValue;
   }
+}
+
+hipError_t launch_dequant_rows_host(const uint32_t* w, const void* scales, const void* biases,
+                                    const int64_t* rows, int count, void* out, int k, int n,
+                                    int dtype, hipStream_t stream) {
+  const size_t row_bytes = (size_t)k * (dtype == kF32 ? 4 : 2);
+  hipError_t e = hipSuccess;
+  for (int r0 = 0; r0 < count && e == hipSuccess; r0 += kArgRows) {
+    const int c = std::min(kArgRows, count - r0);
+    ArgRows src{};
+    for (int i = 0; i < c; ++i) src.ids[i] = (int32_t)rows[r0 + i];
+    char* o = static_cast<char*>(out) + (size_t)r0 * row_bytes;
+    switch (dtype) {
+      case kBf16: e = launch_rows_out<Bf16Out>(w, scales, biases, src, c, o, k, n, stream); break;
+      case kF16: e = launch_rows_out<F16Out>(w, scales, biases, src, c, o, k, n, stream); break;
+      case kF32: e = launch_rows_out<F32Out>(w, scales, biases, src, c, o, k, n, stream); break;
+      default: e = hipErrorInvalidValue;
+    }
+  }
+  return e;
 }
 
 hipError_t launch_dequant(const uint32_t* w, const void* scales, const void* biases, void* out,

@@ -19,6 +19,13 @@ hipError_t launch_dequant_rows(const uint32_t* w, const void* scales, const void
                                const int32_t* rows, int count, void* out, int k, int n, int dtype,
                                hipStream_t stream);
 
+// The same with the ids in host memory, read before this returns (weak: see
+// launch_qgemm_group).
+__attribute__((weak)) hipError_t launch_dequant_rows_host(const uint32_t* w, const void* scales,
+                                                          const void* biases, const int64_t* rows,
+                                                          int count, void* out, int k, int n,
+                                                          int dtype, hipStream_t stream);
+
 // y[m][n] = x . deq(W)^T for 1 <= m <= 16, T in {bf16, f16, f32}; no MFMA.
 hipError_t launch_qgemv(const uint32_t* w, const void* scales, const void* biases, const void* x,
                         void* y, int k, int n, int m, int dtype, hipStream_t stream);
@@ -134,8 +141,8 @@ hipError_t launch_qgemm_swiglu(const uint32_t* w, const void* scales, const void
 // row its own product's.  kStore: y (T) [m, n]; kGateAdd: y (fp32) = residual +
 // gate * float(T(acc)), K split where the plan does and ws holds the partial
 // sums (qgemm_group_split_bytes); kSwiGLU: y (T) [m, width] of n = 2 width
-// weight rows, gate rows first.  (Weak, like every launcher that only step.cpp
-// and cond.cpp call: a host-only build of those leaves it out.)
+// weight rows, gate rows first.  (Weak: a host-only build of the C++ files may
+// leave it out; there is no device to launch on there.)
 struct QgemmGroup {
   enum Stage { kStore, kGateAdd, kSwiGLU };
   struct Product {

@@ -295,27 +295,38 @@ def qmm_gate_add(x, w, scales, biases, residual: torch.Tensor, gate: torch.Tenso
     return out
 
 
+# Host ids past this many are copied to the device in one piece instead.
+MAX_ARG_ROWS = 8 * 768
+
+
 def dequantize_rows(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
                     rows: torch.Tensor, group_size: int = GROUP_SIZE, bits: int = BITS,
                     out: torch.Tensor | None = None) -> torch.Tensor:
     """deq(W)[rows] [len(rows), K] in the scales' dtype: ``DirectTEEncoder.embedRow``
-    (``DirectTEEncoder.swift:106-123``) for a batch of token ids, one launch.
-    Ids are checked against [0, N) here (the kernel clamps them)."""
+    (``DirectTEEncoder.swift:106-123``) for a batch of token ids.  Ids are checked
+    against [0, N); ids on the host go to the kernel as arguments, without a copy
+    to the device (the kernel clamps ids that it reads there)."""
     n, k = _check_weight(w, scales, biases, group_size, bits)
     _require(rows.dim() == 1 and rows.dtype in (torch.int32, torch.int64), "rows: 1-D integer ids")
-    if rows.numel():
-        lo, hi = int(rows.min()), int(rows.max())
-        _require(0 <= lo and hi < n, f"ids must lie in [0, {n}), got [{lo}, {hi}]")
-    ids = rows.to(device=w.device, dtype=torch.int32).contiguous()
+    idx, count = w.get_device(), rows.numel()
+    host = rows.device.type == "cpu" and count <= MAX_ARG_ROWS
+    if host:
+        ids = rows.to(torch.int64).contiguous()
+    else:
+        if count:
+            lo, hi = int(rows.min()), int(rows.max())
+            if not (0 <= lo and hi < n):
+                raise ValueError(f"ids must lie in [0, {n}), got [{lo}, {hi}]")
+        ids = rows.to(device=w.device, dtype=torch.int32).contiguous()
     if out is None:
-        out = torch.empty((ids.numel(), k), dtype=scales.dtype, device=w.device)
-    _require(out.dtype == scales.dtype and out.is_contiguous() and tuple(out.shape) == (ids.numel(), k),
-             f"out must be a contiguous {scales.dtype} [{ids.numel()}, {k}] tensor")
-    ctx = context(w.device)
-    with torch.cuda.device(w.device):
-        st = _lib.load().imq_dequantize_rows(ctx, _ptr(w), _ptr(scales), _ptr(biases), _ptr(ids),
-                                             ids.numel(), _ptr(out), k, n, group_size, bits,
-                                             _DTYPES[scales.dtype], _stream(ids))
+        out = torch.empty((count, k), dtype=scales.dtype, device=w.device)
+    if not (out.dtype == scales.dtype and out.is_contiguous() and out.shape == (count, k)):
+        raise ValueError(f"out must be a contiguous {scales.dtype} [{count}, {k}] tensor")
+    ctx, L = context(idx), _lib.load()
+    fn = L.imq_dequantize_rows_host if host else L.imq_dequantize_rows
+    with torch.cuda.device(idx):
+        st = fn(ctx, _ptr(w), _ptr(scales), _ptr(biases), _ptr(ids), count, _ptr(out), k, n,
+                group_size, bits, _DTYPES[scales.dtype], _stream(out))
     _lib.check(st, ctx)
     return out
 

@@ -118,6 +118,14 @@ int imq_dequantize_rows(imq_ctx* ctx, const uint32_t* w, const void* scales, con
                         const int32_t* rows, int count, void* out, int k, int n, int group_size,
                         int bits, imq_dtype dtype, imq_stream stream);
 
+/* The same with the ids where a tokenizer leaves them: rows int64 [count] in
+ * host memory, read before the call returns and passed as kernel arguments
+ * (no copy to the device; 768 ids a launch).  An id outside [0, N):
+ * IMQ_EINVAL, before any launch. */
+int imq_dequantize_rows_host(imq_ctx* ctx, const uint32_t* w, const void* scales,
+                             const void* biases, const int64_t* rows, int count, void* out, int k,
+                             int n, int group_size, int bits, imq_dtype dtype, imq_stream stream);
+
 /* y[M, N] = x[M, K] . deq(W)^T -- the regime dispatcher.  Replaces the
  * dispatch of `affine_qmm_t_{T}_gs_64_b_4_alN_true_batch_0` in
  * DirectDiTStep.qmm (DirectDiTStep.swift:374-406), DirectTELayerSpike.encodeQmm
