@@ -18,7 +18,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from .ops import Q, _require, context, device_index
+from .ops import Q, _require, context, device_index, raw_stream, run_on
 from .step import _qweight
 
 TIME_L1 = "time_guidance_embed.linear_1"
@@ -45,7 +45,8 @@ class StepConditioning:
 def split_heads(temb: torch.Tensor, heads: torch.Tensor, dim: int) -> StepConditioning:
     """One timestep's temb [dim] and concatenated head outputs [17 dim] as the
     reference's per-step structure (``triples(_:sets:)``, ``:186-197``)."""
-    _require(heads.shape[-1] == 17 * dim, f"heads must be [{17 * dim}] for dim {dim}")
+    if not (heads.shape[-1] == 17 * dim):
+        raise ValueError(f"heads must be [{17 * dim}] for dim {dim}")
 
     def triples(base: int, sets: int):
         return [tuple(heads[base + (3 * i + j) * dim: base + (3 * i + j + 1) * dim]
@@ -136,19 +137,18 @@ class Conditioner:
         if heads is None:
             heads = torch.empty((t.size, self.n_heads), dtype=torch.float32, device=self.device)
         for name, buf, width in (("temb", temb, self.dim), ("heads", heads, self.n_heads)):
-            _require(buf.dtype == torch.float32 and buf.is_contiguous() and buf.device == self.device
-                     and tuple(buf.shape) == (t.size, width),
-                     f"{name} must be a contiguous float32 [{t.size}, {width}] tensor on {self.device}")
-        stream = ctypes.c_void_p(torch.cuda.current_stream(self.device).cuda_stream)
-        with torch.cuda.device(self.device):
-            _lib.check(self._L.imq_cond_step_conditioning(
-                self._h, t.ctypes.data_as(ctypes.c_void_p), t.size, ctypes.c_void_p(temb.data_ptr()),
-                ctypes.c_void_p(heads.data_ptr()), stream), self._ctx)
+            if not (buf.dtype == torch.float32 and buf.is_contiguous() and
+                    buf.device == self.device and tuple(buf.shape) == (t.size, width)):
+                raise ValueError(f"{name} must be a contiguous float32 [{t.size}, {width}] tensor "
+                                 f"on {self.device}")
+        idx = self.device.index
+        _lib.check(run_on(idx, self._L.imq_cond_step_conditioning, self._h, t.ctypes.data, t.size,
+                          temb.data_ptr(), heads.data_ptr(), raw_stream(idx)), self._ctx)
         return temb, heads
 
     def step_conditioning(self, timesteps) -> list[StepConditioning]:
         """``stepConditioning(timesteps:)``: one ``StepConditioning`` per timestep."""
-        _require(self.n_heads == 17 * self.dim,
-                 f"the FLUX.2 heads are 17 dim rows; this chain has {self.n_heads}")
+        if not (self.n_heads == 17 * self.dim):
+            raise ValueError(f"the FLUX.2 heads are 17 dim rows; this chain has {self.n_heads}")
         temb, heads = self.run(timesteps)
         return [split_heads(temb[i], heads[i], self.dim) for i in range(temb.shape[0])]

@@ -63,6 +63,9 @@ def device_index(device: int | str | torch.device | None) -> int:
 def context(device: int | str | torch.device | None = None) -> ctypes.c_void_p:
     """The library context of a HIP device (created once, kept for the process)."""
     idx = device_index(device)
+    ctx = _ctxs.get(idx)
+    if ctx is not None:
+        return ctx
     with _ctx_lock:
         ctx = _ctxs.get(idx)
         if ctx is None:
@@ -74,8 +77,13 @@ def context(device: int | str | torch.device | None = None) -> ctypes.c_void_p:
         return ctx
 
 
+# torch's current stream of a device ordinal as an integer handle, without a
+# Stream object.
+raw_stream = torch._C._cuda_getCurrentRawStream
+
+
 def _stream(t: torch.Tensor) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    return ctypes.c_void_p(raw_stream(t.get_device()))
 
 
 def _ptr(t: torch.Tensor) -> ctypes.c_void_p:
@@ -87,23 +95,42 @@ def _require(cond: bool, msg: str) -> None:
         raise ValueError(msg)
 
 
+def run_on(idx: int, fn, *args) -> int:
+    """fn(*args) with device idx current (the library makes its context's device
+    current; torch's is restored where that is another one)."""
+    if torch.cuda.current_device() == idx:
+        return fn(*args)
+    with torch.cuda.device(idx):
+        return fn(*args)
+
+
+# What a small call costs is mostly here (a projection of one row: about 4 us of
+# library and launch): messages are only formatted when a check fails, pointers
+# and streams go as integers, and no torch object is made but the output
+# (quantized_matmul at one row 15.3 -> 8.2 us of host time).
+
+
 def _check_weight(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
                   group_size: int, bits: int) -> tuple[int, int]:
-    _require(w.is_cuda and scales.is_cuda and biases.is_cuda, "tensors must be on a HIP device")
-    _require(w.dtype in _WORD_DTYPES, f"packed weight must be int32/uint32 words, got {w.dtype}")
-    _require(w.dim() == 2 and scales.dim() == 2 and biases.dim() == 2,
-             "w, scales and biases must be 2-D")
-    _require(w.is_contiguous() and scales.is_contiguous() and biases.is_contiguous(),
-             "w, scales and biases must be contiguous")
-    _require(scales.dtype == biases.dtype, "scales and biases must share a dtype")
+    if not (w.is_cuda and scales.is_cuda and biases.is_cuda):
+        raise ValueError("tensors must be on a HIP device")
+    if w.dtype not in _WORD_DTYPES:
+        raise ValueError(f"packed weight must be int32/uint32 words, got {w.dtype}")
+    wshape, sshape, bshape = w.shape, scales.shape, biases.shape
+    if not len(wshape) == len(sshape) == len(bshape) == 2:
+        raise ValueError("w, scales and biases must be 2-D")
+    if not (w.is_contiguous() and scales.is_contiguous() and biases.is_contiguous()):
+        raise ValueError("w, scales and biases must be contiguous")
+    if scales.dtype != biases.dtype:
+        raise ValueError("scales and biases must share a dtype")
     if group_size != GROUP_SIZE or bits != BITS:
         # the same answer the C ABI gives (IMQ_EUNSUPPORTED)
         raise _lib.ImqUnsupported(_lib.IMQ_EUNSUPPORTED,
                                   f"group_size={group_size} bits={bits}: only 64 / 4 are provided")
-    n, k = w.shape[0], w.shape[1] * 8
-    _require(tuple(scales.shape) == (n, k // GROUP_SIZE) and scales.shape == biases.shape,
-             f"scales/biases must be [{n}, {k // GROUP_SIZE}] for w {tuple(w.shape)}, "
-             f"got {tuple(scales.shape)} / {tuple(biases.shape)}")
+    n, k = wshape[0], wshape[1] * 8
+    if sshape != (n, k // GROUP_SIZE) or sshape != bshape:
+        raise ValueError(f"scales/biases must be [{n}, {k // GROUP_SIZE}] for w {tuple(wshape)}, "
+                         f"got {tuple(sshape)} / {tuple(bshape)}")
     return n, k
 
 
@@ -112,44 +139,51 @@ def dequantize(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
                out: torch.Tensor | None = None) -> torch.Tensor:
     """deq(W) [N, K] in the scales' dtype: RNE(fl32(scale * q + bias)), bit-exact."""
     n, k = _check_weight(w, scales, biases, group_size, bits)
+    idx = w.get_device()
     if out is None:
-        out = torch.empty((n, k), dtype=scales.dtype, device=w.device)
-    _require(out.is_contiguous() and tuple(out.shape) == (n, k) and out.dtype == scales.dtype,
+        out = scales.new_empty((n, k)) if scales.get_device() == idx else \
+            torch.empty((n, k), dtype=scales.dtype, device=w.device)
+    _require(out.is_contiguous() and out.shape == (n, k) and out.dtype == scales.dtype,
              "out must be a contiguous [N, K] tensor of the scales' dtype")
-    dtype = _DTYPES.get(scales.dtype, -1)
-    ctx = context(w.device)
-    with torch.cuda.device(w.device):
-        st = _lib.load().imq_dequantize(ctx, _ptr(w), _ptr(scales), _ptr(biases), _ptr(out),
-                                        k, n, group_size, bits, dtype, _stream(w))
-    _lib.check(st, ctx)
+    ctx = context(idx)
+    _lib.check(run_on(idx, _lib.load().imq_dequantize, ctx, w.data_ptr(), scales.data_ptr(),
+                      biases.data_ptr(), out.data_ptr(), k, n, group_size, bits,
+                      _DTYPES.get(scales.dtype, -1), raw_stream(idx)), ctx)
     return out
+
+
+def _epi_args(x, w, scales, biases, group_size, bits):
+    n, k = _check_weight(w, scales, biases, group_size, bits)
+    if not (x.is_cuda and x.device == w.device):
+        raise ValueError("x must be on the weight's device")
+    xshape = x.shape
+    if not (len(xshape) >= 1 and xshape[-1] == k):
+        raise ValueError(f"x's last dim must be K={k}, got {tuple(xshape)}")
+    if x.dtype != scales.dtype:
+        raise ValueError(f"x ({x.dtype}) and scales ({scales.dtype}) must share T")
+    lead = tuple(xshape[:-1])
+    m = 1
+    for d in lead:
+        m *= d
+    return n, k, m, lead, (x if x.is_contiguous() else x.contiguous())
 
 
 def _qmm_call(entry: str, x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor,
               biases: torch.Tensor, group_size: int, bits: int,
               out: torch.Tensor | None) -> torch.Tensor:
-    n, k = _check_weight(w, scales, biases, group_size, bits)
-    _require(x.is_cuda and x.device == w.device, "x must be on the weight's device")
-    _require(x.dim() >= 1 and x.shape[-1] == k, f"x's last dim must be K={k}, got {tuple(x.shape)}")
-    _require(x.dtype == scales.dtype, f"x ({x.dtype}) and scales ({scales.dtype}) must share T")
-    lead = tuple(x.shape[:-1])
-    m = 1
-    for d in lead:
-        m *= d
-    if not x.is_contiguous():
-        x = x.contiguous()
+    n, k, m, lead, x = _epi_args(x, w, scales, biases, group_size, bits)
+    shape = lead + (n,)
     if out is None:
-        out = torch.empty(lead + (n,), dtype=x.dtype, device=x.device)
-    _require(out.is_contiguous() and tuple(out.shape) == lead + (n,) and out.dtype == x.dtype,
+        out = x.new_empty(shape)
+    _require(out.is_contiguous() and out.shape == shape and out.dtype == x.dtype,
              "out must be a contiguous [..., N] tensor of x's dtype")
     if m == 0:
         return out
-    dtype = _DTYPES.get(x.dtype, -1)
-    ctx = context(w.device)
-    with torch.cuda.device(w.device):
-        st = getattr(_lib.load(), entry)(ctx, _ptr(w), _ptr(scales), _ptr(biases), _ptr(x),
-                                         _ptr(out), k, n, m, group_size, bits, dtype, _stream(x))
-    _lib.check(st, ctx)
+    idx = w.get_device()
+    ctx = context(idx)
+    _lib.check(run_on(idx, getattr(_lib.load(), entry), ctx, w.data_ptr(), scales.data_ptr(),
+                      biases.data_ptr(), x.data_ptr(), out.data_ptr(), k, n, m, group_size, bits,
+                      _DTYPES.get(x.dtype, -1), raw_stream(idx)), ctx)
     return out
 
 
@@ -179,23 +213,11 @@ def qgemm(x, w, scales, biases, group_size: int = GROUP_SIZE, bits: int = BITS, 
     return _qmm_call("imq_qgemm", x, w, scales, biases, group_size, bits, out)
 
 
-def _epi_args(x, w, scales, biases, group_size, bits):
-    n, k = _check_weight(w, scales, biases, group_size, bits)
-    _require(x.is_cuda and x.device == w.device, "x must be on the weight's device")
-    _require(x.dim() >= 1 and x.shape[-1] == k, f"x's last dim must be K={k}, got {tuple(x.shape)}")
-    _require(x.dtype == scales.dtype, f"x ({x.dtype}) and scales ({scales.dtype}) must share T")
-    lead = tuple(x.shape[:-1])
-    m = 1
-    for d in lead:
-        m *= d
-    return n, k, m, lead, (x if x.is_contiguous() else x.contiguous())
-
-
 def _f32_out(out, shape, device, what):
     if out is None:
         return torch.empty(shape, dtype=torch.float32, device=device)
-    _require(out.dtype == torch.float32 and out.is_contiguous() and tuple(out.shape) == shape,
-             f"{what} must be a contiguous float32 tensor of shape {shape}")
+    if not (out.dtype == torch.float32 and out.is_contiguous() and tuple(out.shape) == shape):
+        raise ValueError(f"{what} must be a contiguous float32 tensor of shape {shape}")
     return out
 
 
@@ -207,18 +229,19 @@ def cast_prescale(x: torch.Tensor, scale: float = 16.0, dtype: torch.dtype = tor
     ``scale_dev`` (a one-element float32 device tensor, e.g. ``dynamic_scale``'s)
     replaces ``scale`` and is read when the kernel runs."""
     _require(x.is_cuda and x.dtype == torch.float32, "x must be a float32 HIP tensor")
-    _require(dtype in (torch.float16, torch.bfloat16), f"dtype {dtype}: float16 or bfloat16")
+    if not (dtype in (torch.float16, torch.bfloat16)):
+        raise ValueError(f"dtype {dtype}: float16 or bfloat16")
     x = x if x.is_contiguous() else x.contiguous()
     if out is None:
         out = torch.empty(x.shape, dtype=dtype, device=x.device)
-    _require(out.dtype == dtype and out.is_contiguous() and out.shape == x.shape
-             and out.device == x.device, f"out must be a contiguous {dtype} tensor shaped like x")
+    if not (out.dtype == dtype and out.is_contiguous() and out.shape == x.shape and
+            out.device == x.device):
+        raise ValueError(f"out must be a contiguous {dtype} tensor shaped like x")
     sd = _scale_dev(scale_dev, x.device)
-    ctx = context(x.device)
-    with torch.cuda.device(x.device):
-        st = _lib.load().imq_cast_prescale_ex(ctx, _ptr(x), _ptr(out), x.numel(), float(scale), sd,
-                                              _DTYPES[dtype], _stream(x))
-    _lib.check(st, ctx)
+    idx = x.get_device()
+    ctx = context(idx)
+    _lib.check(run_on(idx, _lib.load().imq_cast_prescale_ex, ctx, x.data_ptr(), out.data_ptr(),
+               x.numel(), float(scale), sd, _DTYPES[dtype], raw_stream(idx)), ctx)
     return out
 
 
@@ -240,11 +263,10 @@ def dynamic_scale(x: torch.Tensor, target: float = 64.0,
     if out is None:
         out = torch.empty(1, dtype=torch.float32, device=x.device)
     _scale_dev(out, x.device)
-    ctx = context(x.device)
-    with torch.cuda.device(x.device):
-        st = _lib.load().imq_dynamic_scale(ctx, _ptr(x), x.numel(), float(target), _ptr(out),
-                                           _stream(x))
-    _lib.check(st, ctx)
+    idx = x.get_device()
+    ctx = context(idx)
+    _lib.check(run_on(idx, _lib.load().imq_dynamic_scale, ctx, x.data_ptr(), x.numel(),
+               float(target), out.data_ptr(), raw_stream(idx)), ctx)
     return out
 
 
@@ -260,17 +282,16 @@ def qmm_postscale(x, w, scales, biases, scale: float, group_size: int = GROUP_SI
     _require(out_dtype in (torch.float32, torch.float16), "out_dtype: float32 or float16")
     if out is None:
         out = torch.empty(lead + (n,), dtype=out_dtype, device=x.device)
-    _require(out.dtype == out_dtype and out.is_contiguous() and tuple(out.shape) == lead + (n,),
-             f"out must be a contiguous {out_dtype} tensor of shape {lead + (n,)}")
+    if not (out.dtype == out_dtype and out.is_contiguous() and tuple(out.shape) == lead + (n,)):
+        raise ValueError(f"out must be a contiguous {out_dtype} tensor of shape {lead + (n,)}")
     sd = _scale_dev(scale_dev, x.device)
     dtype = _DTYPES.get(x.dtype, -1)
-    ctx = context(w.device)
-    with torch.cuda.device(w.device):
-        st = _lib.load().imq_qmm_postscale_ex(ctx, _ptr(w), _ptr(scales), _ptr(biases), _ptr(x),
-                                              _ptr(out), _DTYPES[out_dtype], k, n, m,
-                                              float(scale), sd, group_size, bits, dtype,
-                                              _stream(x))
-    _lib.check(st, ctx)
+    idx = w.get_device()
+    ctx = context(idx)
+    _lib.check(run_on(idx, _lib.load().imq_qmm_postscale_ex, ctx, w.data_ptr(),
+               scales.data_ptr(), biases.data_ptr(), x.data_ptr(), out.data_ptr(),
+               _DTYPES[out_dtype], k, n, m, float(scale), sd, group_size, bits, dtype,
+               raw_stream(idx)), ctx)
     return out
 
 
@@ -286,12 +307,12 @@ def qmm_gate_add(x, w, scales, biases, residual: torch.Tensor, gate: torch.Tenso
              "gate must be float32 [N]")
     out = _f32_out(out, lead + (n,), x.device, "out")
     dtype = _DTYPES.get(x.dtype, -1)
-    ctx = context(w.device)
-    with torch.cuda.device(w.device):
-        st = _lib.load().imq_qmm_gate_add(ctx, _ptr(w), _ptr(scales), _ptr(biases), _ptr(x),
-                                          _ptr(residual), _ptr(gate), _ptr(out), k, n, m,
-                                          float(scale), group_size, bits, dtype, _stream(x))
-    _lib.check(st, ctx)
+    idx = w.get_device()
+    ctx = context(idx)
+    _lib.check(run_on(idx, _lib.load().imq_qmm_gate_add, ctx, w.data_ptr(), scales.data_ptr(),
+               biases.data_ptr(), x.data_ptr(), residual.data_ptr(), gate.data_ptr(),
+               out.data_ptr(), k, n, m, float(scale), group_size, bits, dtype, raw_stream(idx)),
+               ctx)
     return out
 
 
@@ -323,11 +344,10 @@ def dequantize_rows(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
     if not (out.dtype == scales.dtype and out.is_contiguous() and out.shape == (count, k)):
         raise ValueError(f"out must be a contiguous {scales.dtype} [{count}, {k}] tensor")
     ctx, L = context(idx), _lib.load()
-    fn = L.imq_dequantize_rows_host if host else L.imq_dequantize_rows
-    with torch.cuda.device(idx):
-        st = fn(ctx, _ptr(w), _ptr(scales), _ptr(biases), _ptr(ids), count, _ptr(out), k, n,
-                group_size, bits, _DTYPES[scales.dtype], _stream(out))
-    _lib.check(st, ctx)
+    _lib.check(run_on(idx, L.imq_dequantize_rows_host if host else L.imq_dequantize_rows, ctx,
+                      w.data_ptr(), scales.data_ptr(), biases.data_ptr(), ids.data_ptr(), count,
+                      out.data_ptr(), k, n, group_size, bits, _DTYPES[scales.dtype],
+                      raw_stream(idx)), ctx)
     return out
 
 
@@ -343,18 +363,18 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5,
     _require(out_dtype in (torch.bfloat16, torch.float16), "out_dtype: bfloat16 or float16")
     x = x if x.is_contiguous() else x.contiguous()
     cols = x.shape[-1]
-    _require(weight.dtype == torch.float32 and weight.is_contiguous() and weight.numel() == cols
-             and weight.device == x.device, f"weight must be float32 [{cols}] on x's device")
+    if not (weight.dtype == torch.float32 and weight.is_contiguous() and
+            weight.numel() == cols and weight.device == x.device):
+        raise ValueError(f"weight must be float32 [{cols}] on x's device")
     if out is None:
         out = torch.empty(x.shape, dtype=out_dtype, device=x.device)
-    _require(out.dtype == out_dtype and out.is_contiguous() and out.shape == x.shape,
-             f"out must be a contiguous {out_dtype} tensor shaped like x")
-    ctx = context(x.device)
-    with torch.cuda.device(x.device):
-        st = _lib.load().imq_rmsnorm(ctx, _ptr(x), _DTYPES[x.dtype], _ptr(weight), _ptr(out),
-                                     _DTYPES[out_dtype], x.numel() // cols, cols, float(eps),
-                                     _stream(x))
-    _lib.check(st, ctx)
+    if not (out.dtype == out_dtype and out.is_contiguous() and out.shape == x.shape):
+        raise ValueError(f"out must be a contiguous {out_dtype} tensor shaped like x")
+    idx = x.get_device()
+    ctx = context(idx)
+    _lib.check(run_on(idx, _lib.load().imq_rmsnorm, ctx, x.data_ptr(), _DTYPES[x.dtype],
+               weight.data_ptr(), out.data_ptr(), _DTYPES[out_dtype], x.numel() // cols, cols,
+               float(eps), raw_stream(idx)), ctx)
     return out
 
 
@@ -365,19 +385,19 @@ def qmm_add(x, w, scales, biases, residual: torch.Tensor, group_size: int = GROU
     ``DirectGlueKernels.swift:88-96``); residual has x's dtype, ``out=residual``
     updates it in place."""
     n, k, m, lead, x = _epi_args(x, w, scales, biases, group_size, bits)
-    _require(residual.dtype == x.dtype and residual.is_contiguous()
-             and tuple(residual.shape) == lead + (n,), f"residual must be {x.dtype} [..., N]")
+    if not (residual.dtype == x.dtype and residual.is_contiguous() and
+            tuple(residual.shape) == lead + (n,)):
+        raise ValueError(f"residual must be {x.dtype} [..., N]")
     if out is None:
         out = torch.empty(lead + (n,), dtype=x.dtype, device=x.device)
-    _require(out.dtype == x.dtype and out.is_contiguous() and tuple(out.shape) == lead + (n,),
-             f"out must be a contiguous {x.dtype} tensor of shape {lead + (n,)}")
+    if not (out.dtype == x.dtype and out.is_contiguous() and tuple(out.shape) == lead + (n,)):
+        raise ValueError(f"out must be a contiguous {x.dtype} tensor of shape {lead + (n,)}")
     dtype = _DTYPES.get(x.dtype, -1)
-    ctx = context(w.device)
-    with torch.cuda.device(w.device):
-        st = _lib.load().imq_qmm_add(ctx, _ptr(w), _ptr(scales), _ptr(biases), _ptr(x),
-                                     _ptr(residual), _ptr(out), k, n, m, group_size, bits, dtype,
-                                     _stream(x))
-    _lib.check(st, ctx)
+    idx = w.get_device()
+    ctx = context(idx)
+    _lib.check(run_on(idx, _lib.load().imq_qmm_add, ctx, w.data_ptr(), scales.data_ptr(),
+               biases.data_ptr(), x.data_ptr(), residual.data_ptr(), out.data_ptr(), k, n, m,
+               group_size, bits, dtype, raw_stream(idx)), ctx)
     return out
 
 
@@ -400,13 +420,12 @@ def qmm_swiglu(x, w, scales, biases, width: int, gate_row: int, up_row: int,
     else:
         ldy = width
     dtype = _DTYPES.get(x.dtype, -1)
-    ctx = context(w.device)
-    with torch.cuda.device(w.device):
-        st = _lib.load().imq_qmm_swiglu(ctx, _ptr(w), _ptr(scales), _ptr(biases), _ptr(x),
-                                        _ptr(out), ldy, k, n, m, width, gate_row, up_row,
-                                        float(in_scale), float(out_scale), group_size, bits,
-                                        dtype, _stream(x))
-    _lib.check(st, ctx)
+    idx = w.get_device()
+    ctx = context(idx)
+    _lib.check(run_on(idx, _lib.load().imq_qmm_swiglu, ctx, w.data_ptr(), scales.data_ptr(),
+               biases.data_ptr(), x.data_ptr(), out.data_ptr(), ldy, k, n, m, width, gate_row,
+               up_row, float(in_scale), float(out_scale), group_size, bits, dtype,
+               raw_stream(idx)), ctx)
     return out
 
 
@@ -421,7 +440,8 @@ def qmm_plan(m: int, n: int, k: int, dtype: torch.dtype = torch.bfloat16, entry:
     "qgemv", "fused": the post-scale and gated-residual stages over n weight
     rows, "swiglu": n = 2 width) would run for these sizes, without launching
     anything (``imq_qmm_plan``)."""
-    _require(entry in _ENTRIES, f"entry must be one of {sorted(_ENTRIES)}")
+    if not (entry in _ENTRIES):
+        raise ValueError(f"entry must be one of {sorted(_ENTRIES)}")
     ctx = context(device)
     out = _lib.Plan()
     _lib.check(_lib.load().imq_qmm_plan(ctx, _ENTRIES[entry], k, n, m, _DTYPES.get(dtype, -1),
@@ -501,8 +521,8 @@ def apply_linear(linear: QuantizedLinear, x: torch.Tensor, scale: float = 16.0,
     ``linearChunkedSequence`` (``:233-261``) runs this in 512-row chunks to bound MLX
     temporaries; rows are independent, so one launch over all rows gives the same values
     (with the dynamic scale, the reference's chunks would each take their own amax)."""
-    _require(linear.scales.dtype == torch.float16,
-             f"the f16 path needs float16 scales and biases, got {linear.scales.dtype}")
+    if not (linear.scales.dtype == torch.float16):
+        raise ValueError(f"the f16 path needs float16 scales and biases, got {linear.scales.dtype}")
     sd = dynamic_scale(x, dynamic_target) if dynamic_target is not None else None
     x16 = cast_prescale(x, scale, torch.float16, scale_dev=sd)
     return qmm_postscale(x16, linear.weight, linear.scales, linear.biases, scale,

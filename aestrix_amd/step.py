@@ -14,7 +14,7 @@ from dataclasses import dataclass
 import torch
 
 from . import _lib
-from .ops import Q, _DTYPES, context, device_index
+from .ops import Q, _DTYPES, context, device_index, raw_stream, run_on
 from .weights import dit_double_linears, dit_single_linears
 
 
@@ -206,11 +206,10 @@ class DitStep:
     # ---- block halves around the caller's attention (imq_dit_double_attn_in ...)
 
     def _call(self, name: str, *args) -> None:
-        st = torch.cuda.current_stream(self.device).cuda_stream
-        ptrs = [a if isinstance(a, (int, float)) else
-                ctypes.c_void_p(a.data_ptr() if a is not None else 0) for a in args]
-        with torch.cuda.device(self.device):
-            _lib.check(getattr(self._L, name)(self._h, *ptrs, ctypes.c_void_p(st)), self._ctx)
+        idx = self.device.index
+        ptrs = [a if isinstance(a, (int, float)) else (a.data_ptr() if a is not None else 0)
+                for a in args]
+        _lib.check(run_on(idx, getattr(self._L, name), self._h, *ptrs, raw_stream(idx)), self._ctx)
 
     def _joint(self, t: torch.Tensor | None, width: int, dtype: torch.dtype, what: str) -> None:
         if t is None:

@@ -16,7 +16,7 @@ from dataclasses import dataclass
 import torch
 
 from . import _lib
-from .ops import Q, _require, context, device_index
+from .ops import Q, _require, context, device_index, raw_stream, run_on
 from .step import _qweight
 
 # Qwen3 4B text encoder (DirectTEForward.swift:12-22).
@@ -127,9 +127,10 @@ class TextEncoderLayers:
             pass
 
     def _rows(self, x: torch.Tensor, width: int, name: str) -> int:
-        _require(x.dim() == 2 and x.shape[1] == width and x.dtype == self.dtype and x.is_contiguous()
-                 and x.device == self.device,
-                 f"{name} must be a contiguous {self.dtype} [rows, {width}] tensor on {self.device}")
+        if not (x.dim() == 2 and x.shape[1] == width and x.dtype == self.dtype and
+                x.is_contiguous() and x.device == self.device):
+            raise ValueError(f"{name} must be a contiguous {self.dtype} [rows, {width}] tensor "
+                             f"on {self.device}")
         return x.shape[0]
 
     def attn_in(self, layer: int, x: torch.Tensor, qkv: torch.Tensor | None = None) -> torch.Tensor:
@@ -137,13 +138,11 @@ class TextEncoderLayers:
         rows = self._rows(x, self.hidden, "x")
         width = self.nq + 2 * self.nkv
         if qkv is None:
-            qkv = torch.empty((rows, width), dtype=self.dtype, device=self.device)
+            qkv = x.new_empty((rows, width))
         _require(self._rows(qkv, width, "qkv") == rows, "qkv rows must match x")
-        with torch.cuda.device(self.device):
-            _lib.check(self._L.imq_te_attn_in(self._h, layer, ctypes.c_void_p(x.data_ptr()),
-                                              ctypes.c_void_p(qkv.data_ptr()), rows,
-                                              ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)),
-                       self._ctx)
+        idx = self.device.index
+        _lib.check(run_on(idx, self._L.imq_te_attn_in, self._h, layer, x.data_ptr(), qkv.data_ptr(),
+                          rows, raw_stream(idx)), self._ctx)
         return qkv
 
     def attn_out_mlp(self, layer: int, x: torch.Tensor, attn_o: torch.Tensor,
@@ -155,9 +154,7 @@ class TextEncoderLayers:
         if out is None:
             out = torch.empty_like(x)
         _require(self._rows(out, self.hidden, "out") == rows, "out rows must match x")
-        with torch.cuda.device(self.device):
-            _lib.check(self._L.imq_te_attn_out_mlp(
-                self._h, layer, ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(attn_o.data_ptr()),
-                ctypes.c_void_p(out.data_ptr()), rows,
-                ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), self._ctx)
+        idx = self.device.index
+        _lib.check(run_on(idx, self._L.imq_te_attn_out_mlp, self._h, layer, x.data_ptr(),
+                          attn_o.data_ptr(), out.data_ptr(), rows, raw_stream(idx)), self._ctx)
         return out
