@@ -157,14 +157,14 @@ int imq_cond_step_conditioning(imq_cond* c, const float* timesteps, int count, f
     }
     if (e == hipSuccess) e = hipEventRecord(c->copied[half], st);
     float* temb_r = temb + (size_t)r0 * d;
+    // linear_1 and linear_2 with the SiLU after each in their stores.
+    auto f = [](const void* p) { return static_cast<const float*>(p); };
     if (e == hipSuccess)
-      e = imq::launch_qgemv(c->l1.w, c->l1.scales, c->l1.biases, c->sin_dev, c->t1, c->sin_dim, d,
-                            m, IMQ_F32, st);
-    if (e == hipSuccess) e = imq::launch_silu_f32(c->t1, c->t1, m * d, st);
+      e = imq::launch_qgemv_f32_silu(c->l1.w, f(c->l1.scales), f(c->l1.biases), c->sin_dev, nullptr,
+                                     c->t1, c->sin_dim, d, m, st);
     if (e == hipSuccess)
-      e = imq::launch_qgemv(c->l2.w, c->l2.scales, c->l2.biases, c->t1, temb_r, d, d, m, IMQ_F32,
-                            st);
-    if (e == hipSuccess) e = imq::launch_silu_f32(temb_r, c->temb_s, m * d, st);
+      e = imq::launch_qgemv_f32_silu(c->l2.w, f(c->l2.scales), f(c->l2.biases), c->t1, temb_r,
+                                     c->temb_s, d, d, m, st);
     if (e == hipSuccess)
       e = imq::launch_qgemv(c->heads.w, c->heads.scales, c->heads.biases, c->temb_s,
                             heads + (size_t)r0 * c->n_heads, d, c->n_heads, m, IMQ_F32, st);

@@ -30,6 +30,14 @@ __attribute__((weak)) hipError_t launch_dequant_rows_host(const uint32_t* w, con
 hipError_t launch_qgemv(const uint32_t* w, const void* scales, const void* biases, const void* x,
                         void* y, int k, int n, int m, int dtype, hipStream_t stream);
 
+// The f32 qGEMV (1 <= m <= kQgemvMaxM) with v / (1 + exp(-v)) of each output v
+// into y_silu in the store (dd_silu_f32, DirectDiTKernels.swift:176-184); y may be
+// null (weak: see launch_qgemm_group).
+__attribute__((weak)) hipError_t launch_qgemv_f32_silu(const uint32_t* w, const float* scales,
+                                                       const float* biases, const float* x,
+                                                       float* y, float* y_silu, int k, int n, int m,
+                                                       hipStream_t stream);
+
 // The qGEMV with a gate/up pair of weight rows per output (the SwiGLU stage
 // of launch_qgemm_swiglu, same arguments and result) for 1 <= m <=
 // kQgemvSwigluMaxM, T in {bf16, f16}: the gate and up rows of an output are
@@ -188,9 +196,6 @@ hipError_t launch_fill_f32(float* p, float v, int n, hipStream_t stream);
 // (the text encoder's RMSNorm on its T residual stream); T in {bf16, f16}.
 hipError_t launch_rmsnorm_t(const void* x, const float* w, void* y, int rows, int cols, float eps,
                             int dtype, hipStream_t stream);
-
-// y[i] = x[i] / (1 + exp(-x[i])) for i < n, fp32 (y may be x).
-hipError_t launch_silu_f32(const float* x, float* y, int n, hipStream_t stream);
 
 // Largest M the qGEMV kernel takes.
 constexpr int kQgemvMaxM = 16;
