@@ -1,6 +1,7 @@
 // qgemm.hip -- tile plans and launches of the dense quantized matmul (the
 // kernels: qgemm_tile.hpp).
 #include <algorithm>
+#include <type_traits>
 
 #include "epilogue.hpp"
 #include "imq_device.hpp"
@@ -48,16 +49,26 @@ constexpr CostModel kLarge = {
     12.0, 12.0, 3.0, 6.0, 0.0, 8.0 / 1.4e6};
 constexpr size_t kLargeMaxPanel = (size_t)4 << 20;  // of a 128-column tile's activations
 
+// The encoder layers' residual add (K % 256 == 0) keeps the former model past 128
+// rows: an unsplit tile reads its residual behind its last product, where the
+// split's second launch streams it, and a layer's weights are often in the
+// last-level cache, where more splits pay less than the fit has it.  Four layers,
+// fitted against former: 1024 wide, 180 rows 197.9 / 194 us, 511 rows 236.1 / 230.3;
+// 2560 wide, 384 rows 510.5 / 489; below the line 128 rows 1024 wide 186 / 192.
+constexpr int kResidFitRows = 128;
+
 // Tile and K split of a launch over n weight rows (split: K may be split;
 // pair: a gate/up pair, whose wave holds gate and up columns: 256-column tiles
 // of 128 rows and more).  Splits are taken only when the tiles leave CUs idle.
 // ms: the rows of each of `count` products of one launch.
-BigPlan pick_big_plan(const int* ms, int count, int n, int k, int cus, bool split, bool pair) {
+BigPlan pick_big_plan(const int* ms, int count, int n, int k, int cus, bool split, bool pair,
+                      bool resid = false) {
   int m = 0;
   for (int i = 0; i < count; ++i) m += ms[i];
   const int steps = (k + 255) / 256 * 2;  // of 128, whole scale blocks
   const bool tail = k % 256 != 0;
-  const bool large = (size_t)m * n * 8 > kStaticScratchBytes;
+  const bool large = (size_t)m * n * 8 > kStaticScratchBytes ||
+                     (resid && !tail && m > kResidFitRows);
   const CostModel& c = large ? kLarge : kFit;
   BigPlan best{8, 2, 1, steps};
   double best_cost = 1e30;
@@ -100,8 +111,9 @@ BigPlan pick_big_plan(const int* ms, int count, int n, int k, int cus, bool spli
   return best;
 }
 
-BigPlan pick_big_plan(int m, int n, int k, int cus, bool split, bool pair = false) {
-  return pick_big_plan(&m, 1, n, k, cus, split, pair);
+BigPlan pick_big_plan(int m, int n, int k, int cus, bool split, bool pair = false,
+                      bool resid = false) {
+  return pick_big_plan(&m, 1, n, k, cus, split, pair, resid);
 }
 
 // 16-byte alignment of an output or residual pointer (vector output stores).
@@ -158,9 +170,10 @@ hipError_t launch_big_ep(const uint32_t* w, const uint16_t* scales, const uint16
   }
   const bool tail = k % 256 != 0;
   const int cus = device_cus();
-  BigPlan p = pick_big_plan(m, cols, k, cus, ws.p != nullptr, EP::kPair);
+  constexpr bool kResid = std::is_same_v<EP, EpResidAdd<T>>;
+  BigPlan p = pick_big_plan(m, cols, k, cus, ws.p != nullptr, EP::kPair, kResid);
   if (p.splits > 1 && ws.bytes < (size_t)p.splits * m * cols * sizeof(float))
-    p = pick_big_plan(m, cols, k, cus, false, EP::kPair);  // no room for the partial sums
+    p = pick_big_plan(m, cols, k, cus, false, EP::kPair, kResid);  // no room for the partial sums
   if (p.splits == 1)
     return tail ? tile::launch_plan<T, EP, true>(p, w, scales, biases, x, ep, k, n, m, stream)
                 : tile::launch_plan<T, EP, false>(p, w, scales, biases, x, ep, k, n, m, stream);
@@ -205,10 +218,10 @@ hipError_t launch_qgemm(const uint32_t* w, const void* scales, const void* biase
 size_t qgemm_split_bytes(int k, int n, int m, bool fused) {
   if (!qgemm_big_supported(k, n, m)) return 0;
   // The most a stage over these rows takes: a fused stage may be a gate/up
-  // pair (no 128-column tiles) or another.
+  // pair (no 128-column tiles), a residual add or another.
   size_t bytes = 0;
-  for (int v = 0; v < (fused ? 2 : 1); ++v) {
-    const BigPlan p = pick_big_plan(m, n, k, device_cus(), true, v == 1);
+  for (int v = 0; v < (fused ? 3 : 1); ++v) {
+    const BigPlan p = pick_big_plan(m, n, k, device_cus(), true, v == 1, v == 2);
     if (p.splits > 1) bytes = std::max(bytes, (size_t)p.splits * m * n * sizeof(float));
   }
   return bytes;

@@ -66,3 +66,29 @@ def test_split_sums_of_unaligned_rows(m, n, k):
     x = torch.zeros((m, k), dtype=torch.bfloat16, device="cuda")
     x[torch.arange(m), cols] = 1.0
     assert torch.equal(imq.quantized_matmul(x, w, s, b), imq.dequantize(w, s, b)[:, cols].T)
+
+
+@pytest.mark.parametrize("rows", [33, 128, 129, 180, 511])
+@pytest.mark.parametrize("hidden,nq", [(1024, 2048), (576, 3072), (704, 576)])
+def test_layer_residual_add_around_its_plan_line(rows, hidden, nq):
+    """The encoder layers' residual add: two planner models and, at 576, no K split.
+    One-hot attention rows pick single weights of o and a zero down projection adds
+    nothing, so the layer's output is T(x + weight) whatever tiles and splits."""
+    from aestrix_amd.te import TeLayer, TextEncoderLayers
+    print(f"layer residual add rows={rows} hidden={hidden} nq={nq}", flush=True)
+    def proj(n, k, seed):
+        _, w, s, b = problem(1, n, k, "bf16", seed)
+        return imq.Q(w=w, s=s, b=b, n=n, k=k)
+    o, down = proj(hidden, nq, 1), proj(hidden, 512, 2)
+    down.s.zero_(), down.b.zero_()
+    ones = torch.ones(hidden, device="cuda")
+    te = TextEncoderLayers([TeLayer(qkv=proj(nq + 128, hidden, 3), o=o, gate_up=proj(1024, hidden, 4),
+                                    down=down, norm_in=ones, norm_post=ones)], max_rows=512)
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    x = torch.randn((rows, hidden), device="cuda", generator=g).bfloat16()
+    cols = torch.linspace(0, nq - 1, rows).long().cuda()
+    attn = torch.zeros((rows, nq), dtype=torch.bfloat16, device="cuda")
+    attn[torch.arange(rows), cols] = 1.0
+    want = (x.float() + imq.dequantize(o.w, o.s, o.b)[:, cols].T.float()).bfloat16()
+    assert torch.equal(te.attn_out_mlp(0, x, attn), want)
+    te.close()
