@@ -58,7 +58,13 @@ constexpr int max_chunks(int mr) { return mr >= 8 ? 4 : 8; }
 // halved waves cost as much ([9728 x 2560] 12.5 / 12.4), under 768 of K the
 // sums across lanes do ([16384 x 512] 5.1 / 6.8).  From M = 8 the kernel holds two
 // rows already; four spill into too few waves ([20000 x 4096] M = 12 64.5 / 91.9).
-constexpr int kF32WideMinN = 16384, kF32WideMinK = 768;
+// A K tile that leaves lanes of its last chunk idle loses more by it, the doubled
+// registers having halved the waves that hide it: M = 2 [18432 x 2560] (80 of 96
+// chunks) 12.1 / 13.5, [43520 x 2560] 22.5 / 23.4, [18432 x 3584] 16.5 / 18.7, M = 4
+// [20000 x 5120] 32.4 / 34.3, [20000 x 9728] 67.2 / 69.1, M = 3 [26112 x 1536] 13.4 /
+// 14.2; so the two rows are for tiles that fill nine tenths, and from M = 3 on for
+// any tile over enough rows ([30000 x 2560] 24.7 / 23.5, [40000 x 1536] 19.5 / 17.7).
+constexpr int kF32WideMinN = 16384, kF32WideMinK = 768, kF32WideAnyTileN = 28672;
 
 // One K tile of x in LDS, in 16-byte pieces (EPP = 16 / sizeof(T) elements;
 // P = 32 / EPP pieces per chunk of 32 elements): row m, piece p of chunk j
@@ -606,7 +612,9 @@ template <int T, int MR>
 hipError_t launch_m(const uint32_t* w, const void* s, const void* b, const void* x, void* y, int k,
                     int n, int m, const GvPair* pr, hipStream_t stream) {
   if constexpr (T == kF32 && (MR == 2 || MR == 4)) {
-    if (n >= kF32WideMinN && k >= kF32WideMinK)
+    const int tch = tile_len(k, MR, 32, Elem<T>::kBytes) / 32;
+    const bool full = 10 * tch >= 9 * ((tch + 31) / 32 * 32);
+    if (n >= kF32WideMinN && k >= kF32WideMinK && (full || (MR == 4 && n >= kF32WideAnyTileN)))
       return launch_r<T, MR, 2>(w, s, b, x, y, k, n, m, pr, stream);
   }
   return launch_r<T, MR, rows_per_lane(MR)>(w, s, b, x, y, k, n, m, pr, stream);

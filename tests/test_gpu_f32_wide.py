@@ -1,5 +1,6 @@
 """The f32 qGEMV with two weight rows per lane (two to four rows of x, from
-16384 weight rows and K = 768 on) and its neighbours on the one-row form.
+16384 weight rows and K = 768 on, in K tiles that fill the lanes, or over many
+rows) and its neighbours on the one-row form.
 
 Oracle: float64 sums of x with the bit-exact f32 weights.  An fp32 sum of K
 products in any order is off by at most K 2^-23 of the sum of their magnitudes
@@ -25,7 +26,8 @@ def _need_gpu():
 
 @pytest.mark.parametrize("m", [1, 2, 3, 4, 5])
 @pytest.mark.parametrize("n,k", [(16383, 768), (16384, 704), (16384, 768), (16385, 832),
-                                 (16500, 4160), (17000, 3072)])
+                                 (16385, 960), (16500, 4160), (17000, 3072), (17000, 4032),
+                                 (28671, 1536), (28672, 1536)])
 def test_f32_wide_rows(m, n, k):
     print(f"f32 wide M={m} N={n} K={k}", flush=True)
     x, w, s, b = synth.to_device(synth.make_problem(m, n, k, seed=m + k))
