@@ -13,7 +13,7 @@
  * six dependent M = 1 dispatches and a blocking wait each.  Here all
  * timesteps of a call are rows of one pass (every op is row-local), the four
  * heads share one launch over their concatenation along N, and nothing
- * blocks: three matmuls and two SiLU launches per 16 timesteps.
+ * blocks: three matmuls, the SiLU in the stores of two, per 16 timesteps.
  */
 #ifndef IMQ_COND_H
 #define IMQ_COND_H
