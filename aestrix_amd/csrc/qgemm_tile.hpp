@@ -998,12 +998,17 @@ hipError_t launch_big(const BigPlan& p, const uint32_t* w, const uint16_t* scale
 // the output stage ep (its T rounding of value / value2, then emit8 or
 // emit1): 8 consecutive outputs of a row per thread.  Partials of split s
 // sit at ws + s * M * ldp; plain stages read column c at c, pair stages the
-// gate sum at c and the up sum at width + c.  vload: every row and pair offset
-// allows 16-byte partial loads.
-template <int T, class EP>
+// gate sum at c and the up sum at width + c.  VLOAD: 16-byte partial loads
+// (ncols and every row and pair offset multiples of four floats).  Bound by the round trips of the loads: the
+// compiler moves each split's loads to its adds, so a thread waits once per
+// split.  The two forms are kernels of their own: in one, the single floats'
+// clamped columns cost the 16-byte form 28 registers (24 -> 52, a pair's 40 ->
+// 76, past the 64 that eight waves a SIMD have).  Apart, four encoder layers 1024
+// wide take 213.9 / 217.0 / 225.5 us at 384 / 448 / 511 rows (217.7 / 221.6 / 229.1
+// in one), and [200 x 700] K = 2560, whose rows end in half a piece, 10.7 (11.7).
+template <int T, class EP, bool VLOAD>
 __global__ __launch_bounds__(256) void reduce_ep_kernel(const float* __restrict__ ws, int splits,
-                                                        int M, int ncols, int ldp, bool vload,
-                                                        const EP ep) {
+                                                        int M, int ncols, int ldp, const EP ep) {
   const int cpr = (ncols + 7) / 8;
   const long t = (long)blockIdx.x * 256 + threadIdx.x;
   if (t >= (long)M * cpr) return;
@@ -1013,58 +1018,40 @@ __global__ __launch_bounds__(256) void reduce_ep_kernel(const float* __restrict_
   float a[8], u[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) a[e] = u[e] = 0.f;
-  if (vload && c0 + 8 <= ncols) {
-    // The loads of kBatch splits go out before the first add (indices past
-    // the last split repeat it and are not added): one memory round trip per
-    // batch instead of one per split.
-    constexpr int kBatch = EP::kPair ? 4 : 8;
-    for (int s0 = 0; s0 < splits; s0 += kBatch) {
-      float4 p[kBatch][2], q[kBatch][2];
-#pragma unroll
-      for (int j = 0; j < kBatch; ++j) {
-        const float* pr = ws + (size_t)min(s0 + j, splits - 1) * stride + (size_t)row * ldp + c0;
-        p[j][0] = reinterpret_cast<const float4*>(pr)[0];
-        p[j][1] = reinterpret_cast<const float4*>(pr)[1];
-        if constexpr (EP::kPair) {
-          q[j][0] = reinterpret_cast<const float4*>(pr + ep.width)[0];
-          q[j][1] = reinterpret_cast<const float4*>(pr + ep.width)[1];
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < kBatch; ++j) {
-        if (s0 + j >= splits) break;
-        a[0] += p[j][0].x; a[1] += p[j][0].y; a[2] += p[j][0].z; a[3] += p[j][0].w;
-        a[4] += p[j][1].x; a[5] += p[j][1].y; a[6] += p[j][1].z; a[7] += p[j][1].w;
-        if constexpr (EP::kPair) {
-          u[0] += q[j][0].x; u[1] += q[j][0].y; u[2] += q[j][0].z; u[3] += q[j][0].w;
-          u[4] += q[j][1].x; u[5] += q[j][1].y; u[6] += q[j][1].z; u[7] += q[j][1].w;
-        }
+  if constexpr (VLOAD) {
+    // A row's last piece may hold four outputs: its first half twice.
+    const float* p0 = ws + (size_t)row * ldp + c0;
+    const float* p1 = p0 + (c0 + 8 <= ncols ? 4 : 0);
+#pragma unroll 1
+    for (int sp = 0; sp < splits; ++sp, p0 += stride, p1 += stride) {
+      const float4 x = *reinterpret_cast<const float4*>(p0);
+      const float4 y = *reinterpret_cast<const float4*>(p1);
+      a[0] += x.x; a[1] += x.y; a[2] += x.z; a[3] += x.w;
+      a[4] += y.x; a[5] += y.y; a[6] += y.z; a[7] += y.w;
+      if constexpr (EP::kPair) {
+        const float4 z = *reinterpret_cast<const float4*>(p0 + ep.width);
+        const float4 v = *reinterpret_cast<const float4*>(p1 + ep.width);
+        u[0] += z.x; u[1] += z.y; u[2] += z.z; u[3] += z.w;
+        u[4] += v.x; u[5] += v.y; u[6] += v.z; u[7] += v.w;
       }
     }
   } else {
-    // Unaligned rows, or a row's last few outputs (columns past the end repeat
-    // the last one and are not stored): single floats, batched alike.
-    constexpr int kBatch = EP::kPair ? 2 : 4;
-    for (int s0 = 0; s0 < splits; s0 += kBatch) {
-      float p[kBatch][8], q[kBatch][8];
+    // Single floats, eight of a split at once (columns past the end repeat the
+    // last one and are not stored).
+    const float* pr = ws + (size_t)row * ldp;
+#pragma unroll 1
+    for (int sp = 0; sp < splits; ++sp, pr += stride) {
+      float p[8], q[8];
 #pragma unroll
-      for (int j = 0; j < kBatch; ++j) {
-        const float* pr = ws + (size_t)min(s0 + j, splits - 1) * stride + (size_t)row * ldp;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int c = min(c0 + e, ncols - 1);
-          p[j][e] = pr[c];
-          if constexpr (EP::kPair) q[j][e] = pr[ep.width + c];
-        }
+      for (int e = 0; e < 8; ++e) {
+        const int c = min(c0 + e, ncols - 1);
+        p[e] = pr[c];
+        if constexpr (EP::kPair) q[e] = pr[ep.width + c];
       }
 #pragma unroll
-      for (int j = 0; j < kBatch; ++j) {
-        if (s0 + j >= splits) break;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          a[e] += p[j][e];
-          if constexpr (EP::kPair) u[e] += q[j][e];
-        }
+      for (int e = 0; e < 8; ++e) {
+        a[e] += p[e];
+        if constexpr (EP::kPair) u[e] += q[e];
       }
     }
   }
@@ -1110,12 +1097,16 @@ hipError_t tile::launch_sum(const SplitWs& ws, int splits, int m, int ncols, int
                          hipStream_t stream) {
   const long threads = (long)m * ((ncols + 7) / 8);
   const dim3 grid((unsigned)((threads + 255) / 256));
-  // 16-byte partial loads: ws 16-byte aligned and every row / pair offset a
-  // multiple of four floats.
-  bool vload = ldp % 4 == 0 && ((uintptr_t)ws.p & 15u) == 0;
+  // 16-byte partial loads: ws 16-byte aligned, ncols and every row / pair
+  // offset a multiple of four floats.
+  bool vload = ldp % 4 == 0 && ncols % 4 == 0 && ((uintptr_t)ws.p & 15u) == 0;
   if constexpr (EP::kPair) vload = vload && ep.width % 4 == 0;
-  hipLaunchKernelGGL((reduce_ep_kernel<T, EP>), grid, dim3(256), 0, stream, ws.p, splits, m, ncols,
-                     ldp, vload, ep);
+  if (vload)
+    hipLaunchKernelGGL((reduce_ep_kernel<T, EP, true>), grid, dim3(256), 0, stream, ws.p, splits,
+                       m, ncols, ldp, ep);
+  else
+    hipLaunchKernelGGL((reduce_ep_kernel<T, EP, false>), grid, dim3(256), 0, stream, ws.p, splits,
+                       m, ncols, ldp, ep);
   return hipGetLastError();
 }
 
