@@ -19,12 +19,10 @@ hipError_t launch_dequant_rows(const uint32_t* w, const void* scales, const void
                                const int32_t* rows, int count, void* out, int k, int n, int dtype,
                                hipStream_t stream);
 
-// The same with the ids in host memory, read before this returns (weak: see
-// launch_qgemm_group).
-__attribute__((weak)) hipError_t launch_dequant_rows_host(const uint32_t* w, const void* scales,
-                                                          const void* biases, const int64_t* rows,
-                                                          int count, void* out, int k, int n,
-                                                          int dtype, hipStream_t stream);
+// The same with the ids in host memory, read before this returns.
+hipError_t launch_dequant_rows_host(const uint32_t* w, const void* scales, const void* biases,
+                                    const int64_t* rows, int count, void* out, int k, int n,
+                                    int dtype, hipStream_t stream);
 
 // y[m][n] = x . deq(W)^T for 1 <= m <= 16, T in {bf16, f16, f32}; no MFMA.
 hipError_t launch_qgemv(const uint32_t* w, const void* scales, const void* biases, const void* x,
@@ -32,11 +30,10 @@ hipError_t launch_qgemv(const uint32_t* w, const void* scales, const void* biase
 
 // The f32 qGEMV (1 <= m <= kQgemvMaxM) with v / (1 + exp(-v)) of each output v
 // into y_silu in the store (dd_silu_f32, DirectDiTKernels.swift:176-184); y may be
-// null (weak: see launch_qgemm_group).
-__attribute__((weak)) hipError_t launch_qgemv_f32_silu(const uint32_t* w, const float* scales,
-                                                       const float* biases, const float* x,
-                                                       float* y, float* y_silu, int k, int n, int m,
-                                                       hipStream_t stream);
+// null.
+hipError_t launch_qgemv_f32_silu(const uint32_t* w, const float* scales, const float* biases,
+                                 const float* x, float* y, float* y_silu, int k, int n, int m,
+                                 hipStream_t stream);
 
 // The qGEMV with a gate/up pair of weight rows per output (the SwiGLU stage
 // of launch_qgemm_swiglu, same arguments and result) for 1 <= m <=
@@ -149,8 +146,7 @@ hipError_t launch_qgemm_swiglu(const uint32_t* w, const void* scales, const void
 // row its own product's.  kStore: y (T) [m, n]; kGateAdd: y (fp32) = residual +
 // gate * float(T(acc)), K split where the plan does and ws holds the partial
 // sums (qgemm_group_split_bytes); kSwiGLU: y (T) [m, width] of n = 2 width
-// weight rows, gate rows first.  (Weak: a host-only build of the C++ files may
-// leave it out; there is no device to launch on there.)
+// weight rows, gate rows first.
 struct QgemmGroup {
   enum Stage { kStore, kGateAdd, kSwiGLU };
   struct Product {
@@ -168,9 +164,9 @@ struct QgemmGroup {
   Stage stage;
   int width;
 };
-__attribute__((weak)) hipError_t launch_qgemm_group(const QgemmGroup& g, int k, int n, int dtype,
-                                                    hipStream_t stream, SplitWs ws = {});
-__attribute__((weak)) size_t qgemm_group_split_bytes(int k, int n, const int* ms, int count);
+hipError_t launch_qgemm_group(const QgemmGroup& g, int k, int n, int dtype, hipStream_t stream,
+                              SplitWs ws = {});
+size_t qgemm_group_split_bytes(int k, int n, const int* ms, int count);
 
 // y[i] (T) = T(x[i] / scale) for i < count, x fp32; T in {bf16, f16}; with
 // scale_dev the scale is read from device memory when the kernel runs.

@@ -20,6 +20,7 @@
 #include <string>
 #include <vector>
 
+#include "ctx.hpp"
 #include "imq.h"
 #include "imq_step.h"
 #include "imq_weights.h"
@@ -177,6 +178,51 @@ uint64_t walk(const imq_st* st) {
   return sum;
 }
 
+// imq_dequantize_rows_host walks a caller's host array of ids: every refusal
+// that it makes there, and a whole walk (which then finds no device to run on,
+// or the stub's launcher).  The array ends with its last id, so that a read
+// past it shows.
+int row_id_checks() {
+  int n = 0;
+  imq_ctx ctx;
+  ctx.device = 1 << 20;  // no such device
+  const uint32_t w[16] = {};
+  const uint16_t s[4] = {};
+  alignas(16) uint16_t out[4] = {};
+  auto call = [&](const int64_t* ids, int count, void* y, int k, int group, int want,
+                  const char* what) {
+    ++n;
+    const int got = imq_dequantize_rows_host(&ctx, w, s, s, ids, count, y, k, 100, group, 4,
+                                             IMQ_BF16, nullptr);
+    if (got != want) {
+      fprintf(stderr, "fuzz_host: imq_dequantize_rows_host(%s) returned %d, expected %d\n", what,
+              got, want);
+      exit(4);
+    }
+  };
+  for (int count : {1, 2, 767, 768, 769, 5000}) {
+    std::vector<int64_t> ids(count);
+    for (auto& i : ids) i = (int64_t)(rng() % 100);
+    call(ids.data(), count, out, 64, 64, IMQ_EHIP, "good ids");
+    for (int64_t bad : {(int64_t)-1, (int64_t)100, INT64_MIN, INT64_MAX, (int64_t)1 << 32}) {
+      const int64_t was = ids.back();
+      ids.back() = bad;
+      call(ids.data(), count, out, 64, 64, IMQ_EINVAL, "a bad last id");
+      ids.back() = was;
+    }
+    call(ids.data(), count, nullptr, 64, 64, IMQ_EINVAL, "null out");
+    call(ids.data(), count, reinterpret_cast<char*>(out) + 2, 64, 64, IMQ_EINVAL, "out off 16");
+    call(reinterpret_cast<int64_t*>(reinterpret_cast<char*>(ids.data()) + 4), count, out, 64, 64,
+         IMQ_EINVAL, "ids off 8");
+    call(ids.data(), count, out, 60, 64, IMQ_EINVAL, "K = 60");
+    call(ids.data(), count, out, 64, 32, IMQ_EUNSUPPORTED, "groups of 32");
+    call(ids.data(), -count, out, 64, 64, IMQ_EINVAL, "a negative count");
+  }
+  call(nullptr, 1, out, 64, 64, IMQ_EINVAL, "null ids");
+  call(nullptr, 0, nullptr, 64, 64, IMQ_OK, "no ids");
+  return n;
+}
+
 int abi_checks() {
   int n = 0;
   auto expect = [&](int got, int want, const char* what) {
@@ -248,6 +294,9 @@ int abi_checks() {
   }
   if (strlen(imq_last_error(nullptr)) == 0) exit(4);
   for (int st = -3; st < 8; ++st) n += imq_status_string(st) != nullptr;
+  expect(imq_dequantize_rows_host(nullptr, w, s, s, nullptr, 1, y, 64, 1, 64, 4, IMQ_BF16, nullptr),
+         IMQ_EINVAL, "imq_dequantize_rows_host(null ctx)");
+  n += row_id_checks();
   expect(imq_abi_version(), IMQ_ABI_VERSION, "imq_abi_version");
   expect(imq_destroy(nullptr), IMQ_OK, "imq_destroy(null)");
   return n;

@@ -52,7 +52,8 @@ QgemmPlan qgemm_plan(int k, int n, int m, bool, bool, int, bool) {
 }
 bool qgemm_big_supported(int k, int n, int m) {
   return (size_t)m * k * 2 < ((size_t)1 << 31) && (size_t)n * k / 2 < ((size_t)1 << 31) &&
-         k % 256 == 0;
+         (k % 256 == 0 || k >= 640 ||
+          (k >= 320 && (size_t)((m + 127) / 128) * ((n + 255) / 256) < 192));
 }
 hipError_t launch_qgemm_postscale(const uint32_t*, const void*, const void*, const void*, float*,
                                   int, int, int, float, int, hipStream_t, SplitWs, const float*) {
@@ -90,7 +91,6 @@ hipError_t launch_rmsnorm(const float*, const float*, void*, int, int, float, in
   return hipErrorNoDevice;
 }
 hipError_t launch_fill_f32(float*, float, int, hipStream_t) { return hipErrorNoDevice; }
-hipError_t launch_silu_f32(const float*, float*, int, hipStream_t) { return hipErrorNoDevice; }
 hipError_t static_scratch(int, void** out) {
   *out = nullptr;
   return hipErrorNoDevice;
@@ -122,6 +122,18 @@ hipError_t launch_dequant_rows(const uint32_t*, const void*, const void*, const 
                                void*, int, int, int, hipStream_t) {
   return hipErrorNoDevice;
 }
+hipError_t launch_dequant_rows_host(const uint32_t*, const void*, const void*, const int64_t*, int,
+                                    void*, int, int, int, hipStream_t) {
+  return hipErrorNoDevice;
+}
+hipError_t launch_qgemv_f32_silu(const uint32_t*, const float*, const float*, const float*, float*,
+                                 float*, int, int, int, hipStream_t) {
+  return hipErrorNoDevice;
+}
+hipError_t launch_qgemm_group(const QgemmGroup&, int, int, int, hipStream_t, SplitWs) {
+  return hipErrorNoDevice;
+}
+size_t qgemm_group_split_bytes(int, int, const int*, int) { return 0; }
 hipError_t launch_qskinny(const uint32_t*, const void*, const void*, const void*, void*, int, int,
                           int, int, hipStream_t, SplitWs) {
   return hipErrorNoDevice;
