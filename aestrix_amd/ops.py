@@ -77,9 +77,14 @@ def context(device: int | str | torch.device | None = None) -> ctypes.c_void_p:
         return ctx
 
 
+def _current_stream(idx: int) -> int:
+    return torch.cuda.current_stream(idx).cuda_stream
+
+
 # torch's current stream of a device ordinal as an integer handle, without a
-# Stream object.
-raw_stream = torch._C._cuda_getCurrentRawStream
+# Stream object (a torch built without a GPU lacks the name: the loaders and the
+# library's own errors are still to be had there).
+raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", _current_stream)
 
 
 def _stream(t: torch.Tensor) -> ctypes.c_void_p:
