@@ -100,6 +100,14 @@ def _require(cond: bool, msg: str) -> None:
         raise ValueError(msg)
 
 
+def new_out(like: torch.Tensor, shape) -> torch.Tensor:
+    """An output of like's dtype and device: a plain tensor, also where `like` is of a
+    subclass (new_empty would give another of it; torch.empty takes 0.7 us more)."""
+    if type(like) is torch.Tensor:
+        return like.new_empty(shape)
+    return torch.empty(shape, dtype=like.dtype, device=like.device)
+
+
 def run_on(idx: int, fn, *args) -> int:
     """fn(*args) with device idx current (the library makes its context's device
     current; torch's is restored where that is another one)."""
@@ -146,7 +154,7 @@ def dequantize(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
     n, k = _check_weight(w, scales, biases, group_size, bits)
     idx = w.get_device()
     if out is None:
-        out = scales.new_empty((n, k)) if scales.get_device() == idx else \
+        out = new_out(scales, (n, k)) if scales.get_device() == idx else \
             torch.empty((n, k), dtype=scales.dtype, device=w.device)
     _require(out.is_contiguous() and out.shape == (n, k) and out.dtype == scales.dtype,
              "out must be a contiguous [N, K] tensor of the scales' dtype")
@@ -179,7 +187,7 @@ def _qmm_call(entry: str, x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor
     n, k, m, lead, x = _epi_args(x, w, scales, biases, group_size, bits)
     shape = lead + (n,)
     if out is None:
-        out = x.new_empty(shape)
+        out = new_out(x, shape)
     _require(out.is_contiguous() and out.shape == shape and out.dtype == x.dtype,
              "out must be a contiguous [..., N] tensor of x's dtype")
     if m == 0:

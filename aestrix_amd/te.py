@@ -16,7 +16,7 @@ from dataclasses import dataclass
 import torch
 
 from . import _lib
-from .ops import Q, _require, context, device_index, raw_stream, run_on
+from .ops import Q, _require, context, device_index, new_out, raw_stream, run_on
 from .step import _qweight
 
 # Qwen3 4B text encoder (DirectTEForward.swift:12-22).
@@ -138,7 +138,7 @@ class TextEncoderLayers:
         rows = self._rows(x, self.hidden, "x")
         width = self.nq + 2 * self.nkv
         if qkv is None:
-            qkv = x.new_empty((rows, width))
+            qkv = new_out(x, (rows, width))
         _require(self._rows(qkv, width, "qkv") == rows, "qkv rows must match x")
         idx = self.device.index
         _lib.check(run_on(idx, self._L.imq_te_attn_in, self._h, layer, x.data_ptr(), qkv.data_ptr(),
