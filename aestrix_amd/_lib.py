@@ -51,6 +51,7 @@ class Plan(ctypes.Structure):
 
 
 IMQ_ENTRY_QMM_T, IMQ_ENTRY_QGEMM, IMQ_ENTRY_QGEMV, IMQ_ENTRY_FUSED, IMQ_ENTRY_SWIGLU = 0, 1, 2, 3, 4
+DIT_GROUPS = {"qkv": 0, "attn_out": 1, "mlp_in": 2, "mlp_out": 3}
 KERNEL_NAMES = {0: "qgemv", 1: "few_row", 2: "tile", 3: "tile_reg"}
 
 
@@ -124,6 +125,8 @@ SIGNATURES = {
     "imq_dit_step_set_head": ([_p, ctypes.POINTER(QWeight), ctypes.POINTER(QWeight)], _i),
     "imq_dit_step_denoise": ([_p, _p, _p, _p, ctypes.c_float, _i, _p], _i),
     "imq_dit_step_launches": ([_p], _i),
+    "imq_dit_step_kernels": ([_p], _i),
+    "imq_dit_step_group_plan": ([_p, _i, ctypes.POINTER(Plan)], _i),
     "imq_dit_double_attn_in": ([_p, _i, _p, _p, _p, _p, _p, _p], _i),
     "imq_dit_double_attn_out": ([_p, _i, _p, _p, _p], _i),
     "imq_dit_double_mlp": ([_p, _i, _p, _p, _p], _i),

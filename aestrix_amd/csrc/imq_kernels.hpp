@@ -66,9 +66,12 @@ hipError_t launch_qgemv_swiglu_norm(const uint32_t* w, const void* scales, const
 // fp32 scratch for split-K partial sums.  With too few output tiles to fill
 // the chip, the MFMA kernel splits K, writes each split's partial sums here
 // and a second kernel adds them; a null or short workspace runs unsplit.
+// kernels, where given, is raised by every kernel that a call given this
+// launches.
 struct SplitWs {
   float* p = nullptr;
   size_t bytes = 0;
+  int* kernels = nullptr;
 };
 
 // y[m][n] = x . deq(W)^T, any m >= 1, T in {bf16, f16}; MFMA.
@@ -166,7 +169,10 @@ struct QgemmGroup {
 };
 hipError_t launch_qgemm_group(const QgemmGroup& g, int k, int n, int dtype, hipStream_t stream,
                               SplitWs ws = {});
-size_t qgemm_group_split_bytes(int k, int n, const int* ms, int count);
+// The plan of such a launch over `count` products of ms rows: big where one
+// kernel runs them all (otherwise one after the other), splits 1 but for
+// kGateAdd, workspace_bytes for all of the partial sums.
+QgemmPlan qgemm_group_plan(QgemmGroup::Stage stage, int k, int n, const int* ms, int count);
 
 // y[i] (T) = T(x[i] / scale) for i < count, x fp32; T in {bf16, f16}; with
 // scale_dev the scale is read from device memory when the kernel runs.

@@ -158,8 +158,10 @@ hipError_t launch_big_ep(const uint32_t* w, const uint16_t* scales, const uint16
                          SplitWs ws) {
   // Short ragged K (the DiT's x_embedder, K = 128) or operands past 32-bit
   // offsets: the register-staged kernel, one pass.
-  if (!qgemm_big_supported(k, n, m))
+  if (!qgemm_big_supported(k, n, m)) {
+    if (ws.kernels) ++*ws.kernels;
     return tile::launch_reg<T, EP>(w, scales, biases, x, ep, k, n, m, stream);
+  }
   int cols = n;  // weight rows covered
   int width = n, gate_row = 0, up_row = 0;
   if constexpr (EP::kPair) {
@@ -174,6 +176,7 @@ hipError_t launch_big_ep(const uint32_t* w, const uint16_t* scales, const uint16
   BigPlan p = pick_big_plan(m, cols, k, cus, ws.p != nullptr, EP::kPair, kResid);
   if (p.splits > 1 && ws.bytes < (size_t)p.splits * m * cols * sizeof(float))
     p = pick_big_plan(m, cols, k, cus, false, EP::kPair, kResid);  // no room for the partial sums
+  if (ws.kernels) *ws.kernels += p.splits == 1 ? 1 : 2;
   if (p.splits == 1)
     return tail ? tile::launch_plan<T, EP, true>(p, w, scales, biases, x, ep, k, n, m, stream)
                 : tile::launch_plan<T, EP, false>(p, w, scales, biases, x, ep, k, n, m, stream);
@@ -385,6 +388,15 @@ hipError_t launch_qgemm_swiglu(const uint32_t* w, const void* scales, const void
 
 namespace {
 
+// Stages of a group that may split K.
+bool group_splits(QgemmGroup::Stage stage) { return stage == QgemmGroup::kGateAdd; }
+
+bool group_fits(int k, int n, const int* ms, int count) {
+  for (int i = 0; i < count; ++i)
+    if (!qgemm_big_supported(k, n, ms[i])) return false;
+  return true;
+}
+
 template <int T>
 hipError_t launch_group_t(const QgemmGroup& in, int k, int n, hipStream_t stream, SplitWs ws) {
   const int cus = device_cus();
@@ -402,11 +414,10 @@ hipError_t launch_group_t(const QgemmGroup& in, int k, int n, hipStream_t stream
       g.p[i].m = in.p[i].m;
     }
   };
-  // Only the gated residual adds run with K long enough to split.
-  const bool can_split = in.stage == QgemmGroup::kGateAdd && ws.p != nullptr;
-  BigPlan p = pick_big_plan(ms, in.count, cols, k, cus, can_split, pair);
+  BigPlan p = pick_big_plan(ms, in.count, cols, k, cus, group_splits(in.stage) && ws.p, pair);
   if (p.splits > 1 && ws.bytes < (size_t)p.splits * m * cols * sizeof(float))
     p = pick_big_plan(ms, in.count, cols, k, cus, false, pair);
+  if (ws.kernels) *ws.kernels += p.splits == 1 ? 1 : 1 + in.count;
   if (in.stage == QgemmGroup::kStore) {
     tile::Group<EpStore<T>> g{};
     fill(g);
@@ -458,19 +469,20 @@ hipError_t launch_group_t(const QgemmGroup& in, int k, int n, hipStream_t stream
 hipError_t launch_qgemm_group(const QgemmGroup& g, int k, int n, int dtype, hipStream_t stream,
                               SplitWs ws) {
   if (g.count < 1 || g.count > tile::kMaxGroup || k % 256 != 0) return hipErrorInvalidValue;
-  bool fits = true;
-  for (int i = 0; i < g.count; ++i) fits = fits && qgemm_big_supported(k, n, g.p[i].m);
-  if (!fits) {  // operands past 32-bit offsets: one after the other
+  int ms[tile::kMaxGroup];
+  for (int i = 0; i < g.count; ++i) ms[i] = g.p[i].m;
+  if (!group_fits(k, n, ms, g.count)) {  // operands past 32-bit offsets: one after the other
+    const SplitWs count_only{nullptr, 0, ws.kernels};
     hipError_t e = hipSuccess;
     for (int i = 0; i < g.count && e == hipSuccess; ++i) {
       const QgemmGroup::Product& p = g.p[i];
       switch (g.stage) {
         case QgemmGroup::kStore:
-          e = launch_qgemm(p.w, p.scales, p.biases, p.x, p.y, k, n, p.m, dtype, stream);
+          e = launch_qgemm(p.w, p.scales, p.biases, p.x, p.y, k, n, p.m, dtype, stream, count_only);
           break;
         case QgemmGroup::kSwiGLU:
           e = launch_qgemm_swiglu(p.w, p.scales, p.biases, p.x, p.y, g.width, k, n, p.m, g.width, 0,
-                                  g.width, 1.0f, 1.0f, dtype, stream, SplitWs{});
+                                  g.width, 1.0f, 1.0f, dtype, stream, count_only);
           break;
         default:
           e = launch_qgemm_gate_add(p.w, p.scales, p.biases, p.x, p.residual, p.gate,
@@ -487,11 +499,14 @@ hipError_t launch_qgemm_group(const QgemmGroup& g, int k, int n, int dtype, hipS
   }
 }
 
-size_t qgemm_group_split_bytes(int k, int n, const int* ms, int count) {
+QgemmPlan qgemm_group_plan(QgemmGroup::Stage stage, int k, int n, const int* ms, int count) {
+  if (!group_fits(k, n, ms, count)) return QgemmPlan{false, 128, 1, 0, 256};
   int m = 0;
   for (int i = 0; i < count; ++i) m += ms[i];
-  const BigPlan p = pick_big_plan(ms, count, n, k, device_cus(), true, false);
-  return p.splits > 1 ? (size_t)p.splits * m * n * sizeof(float) : 0;
+  const BigPlan p = pick_big_plan(ms, count, n, k, device_cus(), group_splits(stage),
+                                  stage == QgemmGroup::kSwiGLU);
+  return QgemmPlan{true, 32 * p.mt, p.splits,
+                   p.splits > 1 ? (size_t)p.splits * m * n * sizeof(float) : 0, 128 * p.nt};
 }
 
 }  // namespace imq

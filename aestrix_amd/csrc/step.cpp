@@ -42,7 +42,7 @@ struct imq_dit_step {
   hipStream_t cap = nullptr;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
-  int launches = 0;
+  int launches = 0, kernels = 0;  // of the last pass (imq_step.h)
   // The head (loadHead, DirectDiTStep.swift:844-884), once set: x_embedder
   // [dim, C] and proj_out [C, dim] over C latent channels, with buffers of
   // their own (a second arena) and the denoise step's own graph.
@@ -68,15 +68,25 @@ constexpr float kEps = 1e-5f;  // DirectDiTStep.swift:416
 size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 
 // The block halves share this launch bookkeeping: every norm, product and
-// scaling counts in st->launches (a grouped launch as many as it holds), and
-// the first failing call's error is kept.
+// scaling counts in st->launches (a grouped launch as many as it holds) and
+// every kernel in st->kernels, and the first failing call's error is kept.
 struct Enc {
   imq_dit_step* st;
   hipStream_t s;
   hipError_t e = hipSuccess;
-  void ok(hipError_t r, int count = 1) {
+  // One kernel that is not a product.
+  void ok(hipError_t r) {
+    ++st->kernels;
+    products(r, 1);
+  }
+  // `count` products, whose kernels the launcher counted (ws).
+  void products(hipError_t r, int count = 1) {
     st->launches += count;
     if (e == hipSuccess) e = r;
+  }
+  imq::SplitWs ws(imq::SplitWs w) const {
+    w.kernels = &st->kernels;
+    return w;
   }
   void sync(hipError_t r) {
     if (e == hipSuccess) e = r;
@@ -87,7 +97,7 @@ struct Enc {
     g.p[g.count++] = {w.w, w.scales, w.biases, x, y, static_cast<const float*>(y), gate, m};
   }
   void group(const imq::QgemmGroup& g, int k, int n) {
-    ok(imq::launch_qgemm_group(g, k, n, (int)st->dtype, s, st->split), g.count);
+    products(imq::launch_qgemm_group(g, k, n, (int)st->dtype, s, ws(st->split)), g.count);
   }
   static const char* rows(const void* base, int row0, int width) {
     return static_cast<const char*>(base) + (size_t)row0 * width * 2;
@@ -184,12 +194,12 @@ void single_attn_in(Enc& c, int b, const float* x, const void* nx, void* qkv, vo
   const int cw = dim + ffi;
   const imq_qweight* W = &st->w[(size_t)12 * d.n_double + 2 * b];
   const void* n = c.norm(x, nx);
-  c.ok(imq::launch_qgemm(W[0].w, W[0].scales, W[0].biases, n, qkv, dim, 3 * dim, J, T, c.s,
-                         st->split));
-  c.ok(imq::launch_qgemm_swiglu(W[0].w, W[0].scales, W[0].biases, n,
-                                static_cast<char*>(concat) + (size_t)dim * 2, cw, dim,
-                                3 * dim + 2 * ffi, J, ffi, 3 * dim, 3 * dim + ffi, 1.0f, 1.0f, T,
-                                c.s, st->split));
+  c.products(imq::launch_qgemm(W[0].w, W[0].scales, W[0].biases, n, qkv, dim, 3 * dim, J, T, c.s,
+                               c.ws(st->split)));
+  c.products(imq::launch_qgemm_swiglu(W[0].w, W[0].scales, W[0].biases, n,
+                                      static_cast<char*>(concat) + (size_t)dim * 2, cw, dim,
+                                      3 * dim + 2 * ffi, J, ffi, 3 * dim, 3 * dim + ffi, 1.0f, 1.0f,
+                                      T, c.s, c.ws(st->split)));
 }
 
 // Single block b after attention (:616-617): to_out over [attention | MLP]
@@ -200,8 +210,8 @@ void single_attn_out(Enc& c, int b, const void* concat, float* x) {
   const int J = d.l_txt + d.l_img, dim = d.dim, ffi = d.ff_inner, T = (int)st->dtype;
   const imq_qweight* W = &st->w[(size_t)12 * d.n_double + 2 * b];
   const float* g = st->gates + ((size_t)4 * d.n_double + b) * dim;
-  c.ok(imq::launch_qgemm_gate_add(W[1].w, W[1].scales, W[1].biases, concat, x, g, x, dim + ffi,
-                                  dim, J, 1.0f, T, c.s, st->split));
+  c.products(imq::launch_qgemm_gate_add(W[1].w, W[1].scales, W[1].biases, concat, x, g, x,
+                                        dim + ffi, dim, J, 1.0f, T, c.s, c.ws(st->split)));
 }
 
 // Launch every kernel of the blocks on stream s over the plan's residual X,
@@ -230,8 +240,9 @@ void head_embed(Enc& c, const float* lat, float* x) {
   const imq_dit_dims& d = st->d;
   const int T = (int)st->dtype, C = st->lat_ch;
   c.ok(imq::launch_prescale(lat, st->lat16, (size_t)d.l_img * C, 16.0f, T, c.s));
-  c.ok(imq::launch_qgemm_postscale(st->x_emb.w, st->x_emb.scales, st->x_emb.biases, st->lat16,
-                                   x + (size_t)d.l_txt * d.dim, C, d.dim, d.l_img, 16.0f, T, c.s));
+  c.products(imq::launch_qgemm_postscale(st->x_emb.w, st->x_emb.scales, st->x_emb.biases, st->lat16,
+                                         x + (size_t)d.l_txt * d.dim, C, d.dim, d.l_img, 16.0f, T,
+                                         c.s, c.ws({})));
 }
 
 // The head's output half (:947-965): proj_out on nh (the caller's norm_out
@@ -248,9 +259,9 @@ void head_out(Enc& c, const float* x, const void* nh, const float* lat_in, float
                              T, c.s, 1.0f / 16.0f));
     nh = st->nH;
   }
-  c.ok(imq::launch_qgemm_gate_add(st->proj_out.w, st->proj_out.scales, st->proj_out.biases, nh,
-                                  lat_in, st->ones, lat_out, d.dim, C, d.l_img, 0.0f, T, c.s,
-                                  st->split_head, st->euler));
+  c.products(imq::launch_qgemm_gate_add(st->proj_out.w, st->proj_out.scales, st->proj_out.biases,
+                                        nh, lat_in, st->ones, lat_out, d.dim, C, d.l_img, 0.0f, T,
+                                        c.s, c.ws(st->split_head), st->euler));
 }
 
 // One denoise step (encodeDenoiseStep, :908-971) on stream s, the inputs
@@ -282,13 +293,26 @@ void release(imq_dit_step* st) {
   if (st->arena) (void)hipFree(st->arena);
 }
 
+// The plan of a double block's launch of one kind.
+imq::QgemmPlan group_plan(const imq_dit_dims& d, int group) {
+  using G = imq::QgemmGroup;
+  const int ms[6] = {d.l_img, d.l_img, d.l_img, d.l_txt, d.l_txt, d.l_txt};
+  const int two[2] = {d.l_img, d.l_txt};
+  switch (group) {
+    case IMQ_DIT_GROUP_QKV: return imq::qgemm_group_plan(G::kStore, d.dim, d.dim, ms, 6);
+    case IMQ_DIT_GROUP_ATTN_OUT: return imq::qgemm_group_plan(G::kGateAdd, d.dim, d.dim, two, 2);
+    case IMQ_DIT_GROUP_MLP_IN:
+      return imq::qgemm_group_plan(G::kSwiGLU, d.dim, 2 * d.ff_inner, two, 2);
+    default: return imq::qgemm_group_plan(G::kGateAdd, d.ff_inner, d.dim, two, 2);
+  }
+}
+
 // Split-K workspace of the plan: the largest any of its projections takes
 // (fused ones over their weight rows, 2 * ff_inner for a SwiGLU pair).
 size_t split_bytes(const imq_dit_dims& d) {
   const int J = d.l_txt + d.l_img, ffi = d.ff_inner, cw = d.dim + d.ff_inner;
-  const int ms[2] = {d.l_img, d.l_txt};
-  const size_t b = std::max(imq::qgemm_group_split_bytes(d.dim, d.dim, ms, 2),
-                            imq::qgemm_group_split_bytes(ffi, d.dim, ms, 2));
+  const size_t b = std::max(group_plan(d, IMQ_DIT_GROUP_ATTN_OUT).workspace_bytes,
+                            group_plan(d, IMQ_DIT_GROUP_MLP_OUT).workspace_bytes);
   return std::max({b, imq::qgemm_split_bytes(d.dim, 3 * d.dim, J),
                    imq::qgemm_split_bytes(d.dim, 2 * ffi, J, true),
                    imq::qgemm_split_bytes(cw, d.dim, J, true)});
@@ -321,12 +345,12 @@ void expected_shape(const imq_dit_dims& d, int i, int& n, int& k) {
 hipError_t capture(imq_dit_step* st, hipError_t (*enc)(imq_dit_step*, hipStream_t),
                    hipGraph_t* graph, hipGraphExec_t* exec) {
   hipError_t e = hipDeviceSynchronize();
-  st->launches = 0;
+  st->launches = st->kernels = 0;
   if (e == hipSuccess) e = enc(st, st->cap);
   if (e == hipSuccess) e = hipStreamSynchronize(st->cap);
   if (e == hipSuccess) e = hipStreamBeginCapture(st->cap, hipStreamCaptureModeRelaxed);
   if (e == hipSuccess) {
-    st->launches = 0;
+    st->launches = st->kernels = 0;
     const hipError_t r = enc(st, st->cap);
     e = hipStreamEndCapture(st->cap, graph);
     if (e == hipSuccess) e = r;
@@ -471,7 +495,7 @@ int imq_dit_step_run(imq_dit_step* st, const float* h_in, const float* e_in, flo
     if (use_graph) {
       e = hipGraphLaunch(st->exec, s);
     } else {
-      st->launches = 0;
+      st->launches = st->kernels = 0;
       e = encode(st, s);
     }
   }
@@ -565,7 +589,7 @@ int imq_dit_step_denoise(imq_dit_step* st, const float* lat_in, const float* e_i
     if (use_graph) {
       e = hipGraphLaunch(st->dexec, s);
     } else {
-      st->launches = 0;
+      st->launches = st->kernels = 0;
       e = encode_denoise(st, s);
     }
   }
@@ -611,7 +635,7 @@ int imq_dit_double_attn_in(imq_dit_step* st, int block, const float* x, const vo
   if (rc != IMQ_OK) return rc;
   if (!x && !nx) return fail(st->ctx, IMQ_EINVAL, "%s: neither x nor nx given", fn);
   Enc c{st, static_cast<hipStream_t>(stream)};
-  st->launches = 0;
+  st->launches = st->kernels = 0;
   double_attn_in(c, block, x, nx, q, k, v);
   return finish(st, c, fn);
 }
@@ -622,7 +646,7 @@ int imq_dit_double_attn_out(imq_dit_step* st, int block, const void* attn, float
   int rc = check_half(st, fn, block, st ? st->d.n_double : 0, "double", {attn, x}, {});
   if (rc != IMQ_OK) return rc;
   Enc c{st, static_cast<hipStream_t>(stream)};
-  st->launches = 0;
+  st->launches = st->kernels = 0;
   double_attn_out(c, block, attn, x);
   return finish(st, c, fn);
 }
@@ -632,7 +656,7 @@ int imq_dit_double_mlp(imq_dit_step* st, int block, const void* nx, float* x, im
   int rc = check_half(st, fn, block, st ? st->d.n_double : 0, "double", {x}, {nx});
   if (rc != IMQ_OK) return rc;
   Enc c{st, static_cast<hipStream_t>(stream)};
-  st->launches = 0;
+  st->launches = st->kernels = 0;
   double_mlp(c, block, nx, x);
   return finish(st, c, fn);
 }
@@ -644,7 +668,7 @@ int imq_dit_single_attn_in(imq_dit_step* st, int block, const float* x, const vo
   if (rc != IMQ_OK) return rc;
   if (!x && !nx) return fail(st->ctx, IMQ_EINVAL, "%s: neither x nor nx given", fn);
   Enc c{st, static_cast<hipStream_t>(stream)};
-  st->launches = 0;
+  st->launches = st->kernels = 0;
   single_attn_in(c, block, x, nx, qkv, concat);
   return finish(st, c, fn);
 }
@@ -655,7 +679,7 @@ int imq_dit_single_attn_out(imq_dit_step* st, int block, const void* concat, flo
   int rc = check_half(st, fn, block, st ? st->d.n_single : 0, "single", {concat, x}, {});
   if (rc != IMQ_OK) return rc;
   Enc c{st, static_cast<hipStream_t>(stream)};
-  st->launches = 0;
+  st->launches = st->kernels = 0;
   single_attn_out(c, block, concat, x);
   return finish(st, c, fn);
 }
@@ -667,7 +691,7 @@ int imq_dit_head_embed(imq_dit_step* st, const float* lat, float* x, imq_stream 
   int rc = check_half(st, fn, 0, 1, "head", {lat, x}, {});
   if (rc != IMQ_OK) return rc;
   Enc c{st, static_cast<hipStream_t>(stream)};
-  st->launches = 0;
+  st->launches = st->kernels = 0;
   head_embed(c, lat, x);
   return finish(st, c, fn);
 }
@@ -681,13 +705,30 @@ int imq_dit_head_out(imq_dit_step* st, const float* x, const void* nh, const flo
   if (rc != IMQ_OK) return rc;
   if (!x && !nh) return fail(st->ctx, IMQ_EINVAL, "%s: neither x nor nh given", fn);
   Enc c{st, static_cast<hipStream_t>(stream)};
-  st->launches = 0;
+  st->launches = st->kernels = 0;
   c.sync(imq::launch_fill_f32(st->euler, 16.0f * dt, 1, c.s));
   head_out(c, x, nh, lat_in, lat_out);
   return finish(st, c, fn);
 }
 
 int imq_dit_step_launches(const imq_dit_step* st) { return st ? st->launches : 0; }
+
+int imq_dit_step_kernels(const imq_dit_step* st) { return st ? st->kernels : 0; }
+
+int imq_dit_step_group_plan(const imq_dit_step* st, int group, imq_plan* out) {
+  const char* fn = "imq_dit_step_group_plan";
+  if (!st) return fail(nullptr, IMQ_EINVAL, "%s: null step", fn);
+  if (!out) return fail(st->ctx, IMQ_EINVAL, "%s: null output", fn);
+  *out = imq_plan{};
+  if (group < IMQ_DIT_GROUP_QKV || group > IMQ_DIT_GROUP_MLP_OUT)
+    return fail(st->ctx, IMQ_EINVAL, "%s: unknown group %d", fn, group);
+  const int rc = bind_device(st->ctx);
+  if (rc != IMQ_OK) return rc;
+  const imq::QgemmPlan p = group_plan(st->d, group);
+  *out = p.big ? imq_plan{IMQ_KERNEL_TILE, p.tile_rows, p.splits, p.workspace_bytes, p.tile_cols}
+               : imq_plan{IMQ_KERNEL_TILE_REG, 0, 0, 0, 0};
+  return IMQ_OK;
+}
 
 int imq_dit_step_destroy(imq_dit_step* st) {
   if (!st) return IMQ_OK;

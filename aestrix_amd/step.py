@@ -286,4 +286,21 @@ class DitStep:
 
     @property
     def launches(self) -> int:
+        """Norms, projections and scalings of the last pass, whatever launches they
+        share or take."""
         return self._L.imq_dit_step_launches(self._h)
+
+    @property
+    def kernels(self) -> int:
+        """Kernels that the last pass launched."""
+        return self._L.imq_dit_step_kernels(self._h)
+
+    def group_plan(self, group: str) -> dict:
+        """The plan of a double block's shared launch: ``group`` "qkv", "attn_out",
+        "mlp_in" or "mlp_out" (``imq_dit_step_group_plan``)."""
+        out = _lib.Plan()
+        _lib.check(run_on(self.device.index, self._L.imq_dit_step_group_plan, self._h,
+                          _lib.DIT_GROUPS[group], ctypes.byref(out)), self._ctx)
+        return {"kernel": _lib.KERNEL_NAMES[out.kernel], "tile_rows": out.tile_rows,
+                "tile_cols": out.tile_cols, "splits": out.splits,
+                "workspace_bytes": out.workspace_bytes}

@@ -160,10 +160,27 @@ int imq_dit_head_embed(imq_dit_step* step, const float* lat, float* x, imq_strea
 int imq_dit_head_out(imq_dit_step* step, const float* x, const void* nh, const float* lat_in,
                      float* lat_out, float dt, imq_stream stream);
 
-/* Norms, projections and scalings of the last pass encoded (eager run, graph
- * capture, or the last block-half call); projections that share a launch count
- * one each. */
+/* Operations of the last pass encoded (eager run, graph capture, or the last
+ * block-half call): its norms, projections and scalings, whatever launches they
+ * share or take (14 per double block, 4 per single one, 4 for the head). */
 int imq_dit_step_launches(const imq_dit_step* step);
+
+/* Kernels that the same pass launched: a double block's projections of one
+ * kind share one, and a launch that splits K adds one sum per projection. */
+int imq_dit_step_kernels(const imq_dit_step* step);
+
+/* The plan of a double block's shared launches (imq_qmm_plan's struct; the same
+ * for every block): kernel IMQ_KERNEL_TILE where one kernel runs the image and
+ * text projections of the kind, IMQ_KERNEL_TILE_REG where operands past 32-bit
+ * offsets make them run one after the other (tile and splits then unsaid).
+ * IMQ_EINVAL for a null plan or output or an unknown kind. */
+typedef enum imq_dit_group {
+    IMQ_DIT_GROUP_QKV = 0,      /* to_q, to_k, to_v and add_q, add_k, add_v */
+    IMQ_DIT_GROUP_ATTN_OUT = 1, /* to_out and to_add_out, gated residual adds */
+    IMQ_DIT_GROUP_MLP_IN = 2,   /* both linear_in, SwiGLU */
+    IMQ_DIT_GROUP_MLP_OUT = 3   /* both linear_out, gated residual adds */
+} imq_dit_group;
+int imq_dit_step_group_plan(const imq_dit_step* step, int group, imq_plan* out);
 
 int imq_dit_step_destroy(imq_dit_step* step);
 

@@ -220,6 +220,10 @@ public final class DirectDiTStepHIP {
         try ctx.sync()
     }
 
-    /// Kernel launches of the last step encoded.
+    /// Norms, projections and scalings of the last step encoded, whatever
+    /// launches they share or take.
     public var launches: Int { step.map { Int(imq_dit_step_launches($0)) } ?? 0 }
+
+    /// Kernels that the last step encoded launched.
+    public var kernels: Int { step.map { Int(imq_dit_step_kernels($0)) } ?? 0 }
 }

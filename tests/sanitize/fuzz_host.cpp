@@ -284,6 +284,9 @@ int abi_checks() {
          "imq_dit_step_set_conditioning(null)");
   expect(imq_dit_step_destroy(nullptr), IMQ_OK, "imq_dit_step_destroy(null)");
   expect(imq_dit_step_launches(nullptr), 0, "imq_dit_step_launches(null)");
+  expect(imq_dit_step_kernels(nullptr), 0, "imq_dit_step_kernels(null)");
+  expect(imq_dit_step_group_plan(nullptr, IMQ_DIT_GROUP_QKV, &plan), IMQ_EINVAL,
+         "imq_dit_step_group_plan(null)");
   imq_ctx* ctx = nullptr;
   expect(imq_create(0, nullptr), IMQ_EINVAL, "imq_create(null out)");
   const int rc = imq_create(-1, &ctx);  // no device: EHIP (count fails) or EINVAL (out of range)

@@ -133,7 +133,9 @@ hipError_t launch_qgemv_f32_silu(const uint32_t*, const float*, const float*, co
 hipError_t launch_qgemm_group(const QgemmGroup&, int, int, int, hipStream_t, SplitWs) {
   return hipErrorNoDevice;
 }
-size_t qgemm_group_split_bytes(int, int, const int*, int) { return 0; }
+QgemmPlan qgemm_group_plan(QgemmGroup::Stage, int, int, const int*, int) {
+  return QgemmPlan{true, 128, 1, 0, 256};
+}
 hipError_t launch_qskinny(const uint32_t*, const void*, const void*, const void*, void*, int, int,
                           int, int, hipStream_t, SplitWs) {
   return hipErrorNoDevice;
