@@ -346,6 +346,8 @@ def dequantize_rows(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
     host = rows.device.type == "cpu" and count <= MAX_ARG_ROWS
     if host:
         ids = rows.to(torch.int64).contiguous()
+        if ids.data_ptr() % 8:  # ids in the middle of a byte buffer
+            ids = ids.clone()
     else:
         if count:
             lo, hi = int(rows.min()), int(rows.max())

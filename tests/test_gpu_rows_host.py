@@ -62,3 +62,14 @@ def test_host_ids_captured_and_out_of_range():
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+
+
+def test_host_ids_in_the_middle_of_a_byte_buffer():
+    n, k = 300, 256
+    _, w, s, b = synth.to_device(synth.make_problem(1, n, k, seed=6))
+    want = imq.dequantize(w, s, b)
+    for off in (1, 4):
+        buf = bytearray(off) + bytearray(torch.arange(40).numpy().tobytes())
+        ids = torch.frombuffer(buf, dtype=torch.int64, offset=off)
+        print(f"rows by host ids {ids.data_ptr() % 8} bytes past a multiple of 8", flush=True)
+        assert torch.equal(imq.dequantize_rows(w, s, b, ids), want[:40])
