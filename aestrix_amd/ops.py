@@ -329,8 +329,11 @@ def qmm_gate_add(x, w, scales, biases, residual: torch.Tensor, gate: torch.Tenso
     return out
 
 
-# Host ids past this many are copied to the device in one piece instead.
-MAX_ARG_ROWS = 8 * 768
+# Host ids past this many are copied to the device in one piece instead: that costs
+# about the same at any count, the arguments one launch per 768 (2560 wide, us a
+# call, copied / as arguments: 30 ids 31.9 / 13.5, 3072 38.1 / 26.4, 4608 38.4 / 35.1,
+# 6144 39.5 / 42.8, 12288 46.9 / 74.5).
+MAX_ARG_ROWS = 6 * 768
 
 
 def dequantize_rows(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
