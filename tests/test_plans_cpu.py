@@ -1,0 +1,57 @@
+"""Tile plans on the host: the planner of qgemm.hip compiled without a device (it
+counts on 256 CUs then) and asked for the plans that a measurement decided."""
+
+from __future__ import annotations
+
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "aestrix_amd", "csrc")
+SOURCE = r"""
+#include "qgemm.hip"
+#include <cstdio>
+int main() {
+  int m, n, k, split, pair, resid;
+  while (std::scanf("%d %d %d %d %d %d", &m, &n, &k, &split, &pair, &resid) == 6) {
+    const imq::BigPlan p = imq::pick_big_plan(m, n, k, 256, split, pair, resid);
+    std::printf("%d %d %d %d\n", 32 * p.mt, 128 * p.nt, p.splits,
+                imq::qgemm_big_supported(k, n, m) ? 1 : 0);
+  }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def plans(tmp_path_factory):
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("no hipcc")
+    d = tmp_path_factory.mktemp("plans")
+    src, exe = d / "plans.hip", d / "plans"
+    src.write_text(SOURCE)
+    # The kernels' launches stay undefined: nothing here calls them.
+    subprocess.run([hipcc, "--offload-host-only", "-std=c++17", "-O1", "-w", "-I", CSRC, "-I",
+                    os.path.join(ROOT, "include"), str(src), "-o", str(exe),
+                    "-Wl,--unresolved-symbols=ignore-all"], check=True, timeout=300)
+
+    def ask(*shapes):
+        text = "\n".join(" ".join(str(int(v)) for v in s) for s in shapes)
+        out = subprocess.run([str(exe)], input=text, capture_output=True, text=True, check=True,
+                             timeout=60, env={**os.environ, "HIP_VISIBLE_DEVICES": ""}).stdout
+        rows = [tuple(int(v) for v in line.split()) for line in out.splitlines()]
+        assert len(rows) == len(shapes)
+        return rows
+
+    return ask
+
+
+def test_ragged_rows_of_partial_sums_split_less(plans):
+    """N % 4 != 0: a split's partial sums are added float by float."""
+    odd, even = plans((62, 12390, 8448, 1, 0, 0), (62, 12392, 8448, 1, 0, 0))
+    assert odd[2] <= 2 < even[2], (odd, even)
+    for s in ((391, 9998, 3712), (372, 6779, 5824)):
+        assert plans((*s, 1, 0, 0))[0][2] == 1, s
