@@ -33,11 +33,15 @@ namespace {
 // both pick alike, and the shapes that the allocation-free entry refuses stay
 // the same.  Below that size a split's partial sums fit that scratch.
 //
-// The fit, made on plain products of aligned widths, lacks a charge: rows of
-// partial sums that are not whole 16-byte pieces (N % 4 != 0) are added float by
-// float.  Without ragged_output [62 x 12390] K = 8448 was split in five, 37.9 us a
+// Two charges that the fit, made on plain products of aligned widths, lacks.  Rows
+// of partial sums that are not whole 16-byte pieces (N % 4 != 0) are added float by
+// float: without ragged_output [62 x 12390] K = 8448 was split in five, 37.9 us a
 // call against 31.3 by two splits; [391 x 9998] K = 3712 68.4 / 50.9, [372 x 6779] K =
-// 5824 57.3 / 45.6; the other way [711 x 2474] K = 9984 52.3 / 55.1.
+// 5824 57.3 / 45.6; the other way [711 x 2474] K = 9984 52.3 / 55.1.  A gate/up pair's
+// sum reads two rows per split: four encoder layers (19456 rows of weights, K =
+// 2560) of 129 / 136 / 144 rows 338.1 / 340.4 / 342.5 us split in three, 330.1 / 330.7 /
+// 332.9 in two; at 64 rows, on half the tile height, three stay ahead, 253.9 against
+// 257.0.
 struct CostModel {
   double step2[9], step1[9];  // per K-step, by mt: 256 and 128 columns
   double round2, round1;      // per round of tiles
@@ -45,15 +49,16 @@ struct CostModel {
   double per_split;           // and per split of it
   double per_output;          // per output and split
   double ragged_output;       // more where rows of partial sums are not whole 16-byte pieces
+  double pair_split;          // a gate/up pair's, per split past the second and 32 rows of tile
 };
 constexpr CostModel kFit = {
     {0, 0.782, 0.967, 0, 1.477, 1.767, 2.102, 2.449, 2.614},
     {0, 0, 0.557, 0, 0.840, 0.978, 1.211, 1.398, 1.512},
-    3.878, 2.818, 2.975, 2.975, 0.371, 1.11e-6, 0.7e-6};
+    3.878, 2.818, 2.975, 2.975, 0.371, 1.11e-6, 0.7e-6, 0.085};
 constexpr CostModel kLarge = {
     {0, 2.5, 3.5, 0, 5.5, 6.5, 7.5, 8.5, 9.5},
     {0, 0, 1.5, 0, 3.35, 4.275, 5.2, 6.125, 7.05},
-    12.0, 12.0, 3.0, 6.0, 0.0, 8.0 / 1.4e6, 0.0};
+    12.0, 12.0, 3.0, 6.0, 0.0, 8.0 / 1.4e6, 0.0, 0.0};
 constexpr size_t kLargeMaxPanel = (size_t)4 << 20;  // of a 128-column tile's activations
 
 // The encoder layers' residual add (K % 256 == 0) keeps the former model past 128
@@ -108,7 +113,8 @@ BigPlan pick_big_plan(const int* ms, int count, int n, int k, int cus, bool spli
         double cost = (double)rounds *
                       (sps * (nt == 2 ? c.step2[mt] : c.step1[mt]) + (nt == 2 ? c.round2 : c.round1));
         if (eff > 1)
-          cost += (nt == 2 ? c.split2 : c.split1) + eff * (c.per_split + (double)m * n * per_output);
+          cost += (nt == 2 ? c.split2 : c.split1) + eff * (c.per_split + (double)m * n * per_output) +
+                  (pair && eff > 2 ? (eff - 2) * mt * c.pair_split : 0.0);
         if (cost < best_cost - 1e-9) {
           best_cost = cost;
           best = BigPlan{mt, nt, eff, sps};

@@ -55,3 +55,13 @@ def test_ragged_rows_of_partial_sums_split_less(plans):
     assert odd[2] <= 2 < even[2], (odd, even)
     for s in ((391, 9998, 3712), (372, 6779, 5824)):
         assert plans((*s, 1, 0, 0))[0][2] == 1, s
+
+
+PAIR_SPLITS = {33: 3, 48: 3, 64: 3, 112: 2, 128: 2, 129: 2, 136: 2, 144: 2, 160: 2, 170: 1}
+
+
+@pytest.mark.parametrize("rows", sorted(PAIR_SPLITS))
+def test_a_gate_up_pairs_third_split(plans, rows):
+    """Four layers (19456 rows of weights, K = 2560) at 129-144 rows: 330-333 us with two
+    splits, 338-343 with three; at 33-64 rows three are ahead."""
+    assert plans((rows, 19456, 2560, 1, 1, 0))[0][2] == PAIR_SPLITS[rows]
