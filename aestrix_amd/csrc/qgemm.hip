@@ -144,21 +144,49 @@ int device_cus() {
   return cus;
 }
 
-// K % 256 != 0: a short K whose 128 x 256 tiles nearly fill
-// the chip stays on the register-staged kernel.  The large-M kernel computes K
-// rounded up to 256, and at three to ten groups its prologue and staged output
-// weigh as much as its loop, while two 128 x 256 workgroups fit a CU.  Measured
-// against it (us, weights past the last-level cache): [4608 x 9216] K = 448 /
-// 576 / 704 / 832 55.0 / 66.4 / 77.2 / 86.1 here, 59.2 / 71.6 / 74.0 / 88.0
-// there; [512 x 18432] K = 320 / 448 / 704 13.4 / 16.5 / 24.9 and 15.9 / 16.8
-// / 20.4; with fewer tiles it has no K split and leaves CUs idle: [2048 x
+// K % 256 != 0: a short K whose 128 x 256 tiles nearly fill the chip stays on the
+// register-staged kernel.  The large-M kernel computes K rounded up to 256, and at
+// three to ten groups its prologue and staged output weigh as much as its loop,
+// while two 128 x 256 workgroups fit a CU.  Measured against it (us, weights past
+// the last-level cache): [4608 x 9216] K = 448 / 576 / 704 55.0 / 66.4 / 77.2 here,
+// 59.2 / 71.6 / 74.0 there; [512 x 18432] K = 320 / 448 / 704 13.4 / 16.5 / 24.9 and
+// 15.9 / 16.8 / 20.4; with fewer tiles it has no K split and leaves CUs idle: [2048 x
 // 2048] K = 320 10.5 and 8.3, [100 x 3072] K = 448 12.2 and 5.6, [333 x 5001]
-// K = 2880 84.5 and 24.3, [512 x 2560] K = 2880 69.1 and 17.3.  Below 320 (one
-// or two blocks) it always stays there.
+// K = 2880 84.5 and 24.3, [512 x 2560] K = 2880 69.1 and 17.3.  At one scale block (K
+// = 64, 128 or 192) it always stays there.
+//
+// From 640 to 1700 of K it stays there where the two costs (us) say so: its tiles
+// just fill one or more rounds of two per CU while the large-M kernel's last round
+// is nearly empty or a quarter of its K is padding.  Both costs are fitted to 430
+// ragged shapes (plain, post-scaled and gate/up outputs alike, so that one choice
+// serves all of them): [865 x 16768] K = 832 / 1152 / 1600 (462 tiles of 128 x 256)
+// 35.9 / 46.7 / 62.0 here, 40.7 / 48.4 / 66.4 there, with post-scaled fp32 outputs 41.7
+// / 52.2 / 67.7 and 50.1 / 57.1 / 72.0; [1948 x 19724] K = 832 125 and 141; on the
+// other side [495 x 26496] K = 1152 45.0 and 40.9, [4608 x 3072] K = 960 35.5 and 33.3.
+// Past 1700 the large-M kernel is level or ahead ([865 x 16768] K = 2112 83.2 and
+// 89.5, but 2880 120.8 and 110.8).
 bool tail_on_register_kernel(int k, int n, int m) {
   if (k % 256 == 0) return false;
   const size_t tiles = (size_t)((m + 127) / 128) * ((n + 255) / 256);
-  return k < 320 || (k < 640 && tiles >= 192);
+  if (k < 320 || (k < 640 && tiles >= 192)) return true;
+  if (k < 640 || k > 1700) return false;
+  const int cus = device_cus();
+  const double outputs = (double)m * n;
+  const BigPlan p = pick_big_plan(m, n, k, cus, false);
+  const size_t big_tiles =
+      (size_t)((m + 32 * p.mt - 1) / (32 * p.mt)) * ((n + 128 * p.nt - 1) / (128 * p.nt));
+  const double rounds = (double)((big_tiles + cus - 1) / cus);
+  const double big =
+      rounds * (1.14 * p.split_steps * (p.nt == 2 ? kFit.step2[p.mt] : kFit.step1[p.mt]) +
+                2.0 * (p.nt == 2 ? kFit.round2 : kFit.round1)) +
+      0.12e-6 * outputs;
+  // Rounds of two workgroups a CU; a last round of one a CU is quicker.
+  const int groups = k / 64;
+  const size_t pairs = tiles / (2 * (size_t)cus), rest = tiles % (2 * (size_t)cus);
+  const double reg = (double)(pairs + (rest > (size_t)cus)) * (1.97 * groups + 0.8) +
+                     (rest > 0 && rest <= (size_t)cus ? 1.54 * groups + 2.7 : 0.0) +
+                     0.55e-6 * outputs;
+  return reg < 1.02 * big;
 }
 
 // The tile kernels with output stage ep (the large-M one with two groups per

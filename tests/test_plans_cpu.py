@@ -65,3 +65,16 @@ def test_a_gate_up_pairs_third_split(plans, rows):
     """Four layers (19456 rows of weights, K = 2560) at 129-144 rows: 330-333 us with two
     splits, 338-343 with three; at 33-64 rows three are ahead."""
     assert plans((rows, 19456, 2560, 1, 1, 0))[0][2] == PAIR_SPLITS[rows]
+
+
+# m, n, k, and whether the large-M kernel takes the shape (else the register-staged).
+RAGGED = [(865, 16768, 704, 0), (865, 16768, 832, 0), (865, 16768, 1152, 0), (865, 16768, 1600, 0),
+          (865, 16768, 2880, 1), (865, 16768, 1280, 1), (1948, 19724, 832, 0),
+          (495, 26496, 1152, 1), (4608, 3072, 960, 1), (333, 5001, 2880, 1), (333, 5001, 704, 1),
+          (2048, 2048, 832, 1), (1500, 12288, 832, 1), (700, 27648, 832, 1), (512, 2560, 320, 1),
+          (512, 18432, 448, 0), (4608, 9216, 192, 0), (64, 512, 64, 0)]
+
+
+@pytest.mark.parametrize("m,n,k,tile", RAGGED)
+def test_kernel_of_a_ragged_k(plans, m, n, k, tile):
+    assert plans((m, n, k, 0, 0, 0))[0][3] == tile
