@@ -553,8 +553,8 @@ int imq_qmm_plan(imq_ctx* ctx, int entry, int k, int n, int m, imq_dtype dtype, 
   int rc = bind_device(ctx);
   if (rc != IMQ_OK) return rc;
   const bool w_fits_gemv = (size_t)n * (size_t)k / 2 < ((size_t)1 << 32);
-  auto tile = [&](bool fused, bool split, bool pair = false) {
-    const imq::QgemmPlan p = imq::qgemm_plan(k, n, m, fused, split, 0, pair);
+  auto tile = [&](bool split, bool pair = false) {
+    const imq::QgemmPlan p = imq::qgemm_plan(k, n, m, split, pair);
     *out = imq_plan{p.big ? IMQ_KERNEL_TILE : IMQ_KERNEL_TILE_REG, p.tile_rows, p.splits,
                     p.workspace_bytes, p.tile_cols};
     return IMQ_OK;
@@ -574,7 +574,7 @@ int imq_qmm_plan(imq_ctx* ctx, int entry, int k, int n, int m, imq_dtype dtype, 
         *out = imq_plan{IMQ_KERNEL_QGEMV, 0, 1, 0};
         return IMQ_OK;
       }
-      return tile(true, false, true);
+      return tile(false, true);
     case IMQ_ENTRY_QGEMM:
     case IMQ_ENTRY_FUSED:
       if (dtype == IMQ_F32) return fail(ctx, IMQ_EUNSUPPORTED, "%s: f32 has no MFMA kernel", fn);
@@ -594,7 +594,7 @@ int imq_qmm_plan(imq_ctx* ctx, int entry, int k, int n, int m, imq_dtype dtype, 
         return IMQ_OK;
       }
       if (dtype == IMQ_F32) return fail(ctx, IMQ_EUNSUPPORTED, "%s: f32 weights of 4 GiB", fn);
-      return tile(false, true);
+      return tile(true);
     }
     default:
       return fail(ctx, IMQ_EINVAL, "%s: unknown entry %d", fn, entry);

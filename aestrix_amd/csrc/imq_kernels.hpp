@@ -85,10 +85,9 @@ size_t qgemm_split_bytes(int k, int n, int m, bool fused = false);
 
 // The plan launch_qgemm / the fused launchers choose: big = the buffer-load
 // MFMA kernel (else the register-staged 128 x 256 tile kernel), its tile
-// height in rows, its K splits and their fp32 workspace bytes.  fused: an
-// output stage other than the plain store over n weight rows (2 * width for a
-// SwiGLU pair); split: a workspace is available; cus: the compute units the
-// planner counts on (0: the device's); pair: the stage is a gate/up pair.
+// height in rows, its K splits and their fp32 workspace bytes.  split: a
+// workspace is available; pair: the stage is a gate/up pair (n = 2 * width
+// weight rows).  The residual add may run another plan (kResidFitRows).
 struct QgemmPlan {
   bool big;
   int tile_rows;
@@ -96,7 +95,7 @@ struct QgemmPlan {
   size_t workspace_bytes;
   int tile_cols;
 };
-QgemmPlan qgemm_plan(int k, int n, int m, bool fused, bool split, int cus, bool pair = false);
+QgemmPlan qgemm_plan(int k, int n, int m, bool split, bool pair);
 
 // Whether the buffer-load MFMA kernel (and so the fused epilogues) takes
 // these shapes: x and w addressable with 32-bit byte offsets, K % 64 == 0 but

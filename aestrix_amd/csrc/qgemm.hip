@@ -272,9 +272,9 @@ size_t qgemm_split_bytes(int k, int n, int m, bool fused) {
   return bytes;
 }
 
-QgemmPlan qgemm_plan(int k, int n, int m, bool, bool split, int cus, bool pair) {
+QgemmPlan qgemm_plan(int k, int n, int m, bool split, bool pair) {
   if (!qgemm_big_supported(k, n, m)) return QgemmPlan{false, 128, 1, 0, 256};
-  const BigPlan p = pick_big_plan(m, n, k, cus > 0 ? cus : device_cus(), split, pair);
+  const BigPlan p = pick_big_plan(m, n, k, device_cus(), split, pair);
   return QgemmPlan{true, 32 * p.mt, p.splits,
                    p.splits > 1 ? (size_t)p.splits * m * n * sizeof(float) : 0, 128 * p.nt};
 }
@@ -430,7 +430,12 @@ hipError_t launch_qgemm_swiglu(const uint32_t* w, const void* scales, const void
 
 namespace {
 
-// Stages of a group that may split K.
+// Stages of a group that may split K: the sums of six q, k and v products would be
+// six more launches, and the split form of a pair's shared launch is not built.
+// Unsplit they are ahead of the separate, split products at every size measured,
+// the smallest blocks too: q, k and v of 256 + 16 rows (dim 1536, 108 tiles on 256
+// CUs) and of 64 + 64 (768) 14.4 and 9.3 us, whole steps of such double blocks by
+// graph 642 -> 425 us (five blocks) and 400 -> 232 (four).
 bool group_splits(QgemmGroup::Stage stage) { return stage == QgemmGroup::kGateAdd; }
 
 bool group_fits(int k, int n, const int* ms, int count) {

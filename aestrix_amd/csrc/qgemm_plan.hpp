@@ -8,8 +8,8 @@
 namespace imq {
 
 // Tile height (32 mt rows), width (128 nt columns) and K split of a launch of
-// the large-M kernel; split_steps K-steps of 128 per split, an even
-// number (K % 256 == 0) or all of them.
+// the large-M kernel; split_steps K-steps of 128 per split, an even number (whole
+// scale blocks, K rounded up to 256).
 struct BigPlan {
   int mt, nt, splits, split_steps;
 };

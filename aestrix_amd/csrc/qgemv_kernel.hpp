@@ -58,12 +58,16 @@ constexpr int max_chunks(int mr) { return mr >= 8 ? 4 : 8; }
 // halved waves cost as much ([9728 x 2560] 12.5 / 12.4), under 768 of K the
 // sums across lanes do ([16384 x 512] 5.1 / 6.8).  From M = 8 the kernel holds two
 // rows already; four spill into too few waves ([20000 x 4096] M = 12 64.5 / 91.9).
-// A K tile that leaves lanes of its last chunk idle loses more by it, the doubled
-// registers having halved the waves that hide it: M = 2 [18432 x 2560] (80 of 96
-// chunks) 12.1 / 13.5, [43520 x 2560] 22.5 / 23.4, [18432 x 3584] 16.5 / 18.7, M = 4
-// [20000 x 5120] 32.4 / 34.3, [20000 x 9728] 67.2 / 69.1, M = 3 [26112 x 1536] 13.4 /
-// 14.2; so the two rows are for tiles that fill nine tenths, and from M = 3 on for
-// any tile over enough rows ([30000 x 2560] 24.7 / 23.5, [40000 x 1536] 19.5 / 17.7).
+// The rule's K tiles that fill 32 lanes nine tenths are those that both forms plan
+// on 32 lanes.  The others run on 16 (make_plan), where a wave's four row groups
+// read the same pieces of x and one row is not bound as above ([52224 x 3072] M = 4
+// put on 16 lanes: 48.2 us by one row, 43.4 by two; on 32 lanes 53.3 / 42.6), and two
+// rows there gain nothing before the rows are many: M = 2 [18432 x 2560] 12.1-13.3 /
+// 13.5, [18432 x 3584] 16.5 / 18.7, [43520 x 2560] level, M = 4 [18432 x 2560] 17.8 / 18.0,
+// [20000 x 5120] 32.4-34.2 / 34.3, M = 3 [26112 x 1536] 13.4-14.4 / 14.2-14.9.  From M = 3
+// and 28672 rows on they do: [30000 x 2560] 25.3 / 23.4, [40000 x 1536] 20.4 / 18.8, [40000
+// x 3584] 42.8 / 37.7.  (The rule asks for 32 lanes also where IMQ_QGEMV_LANES forces
+// another count.)
 constexpr int kF32WideMinN = 16384, kF32WideMinK = 768, kF32WideAnyTileN = 28672;
 
 // One K tile of x in LDS, in 16-byte pieces (EPP = 16 / sizeof(T) elements;

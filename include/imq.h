@@ -167,7 +167,9 @@ int imq_qmm_t(imq_ctx* ctx, const uint32_t* w, const void* scales, const void* b
  * blocking the host, for the previous one on that GPU, whatever its stream,
  * context or thread).  Calls made under stream capture are not: a graph
  * replay that overlaps another call using the scratch on that GPU races and
- * may return wrong results; order such replays on one stream. */
+ * may return wrong results; order such replays on one stream.  The calls that
+ * use it are those whose imq_qmm_plan has workspace_bytes > 0; a K that is not a
+ * multiple of 256 may be among them (from K = 320). */
 int imq_qmm_t_noalloc(imq_ctx* ctx, const uint32_t* w, const void* scales, const void* biases,
                       const void* x, void* y, int k, int n, int m, int group_size, int bits,
                       imq_dtype dtype, imq_stream stream);
@@ -197,16 +199,18 @@ typedef enum imq_entry {
     IMQ_ENTRY_QMM_T = 0,   /* imq_qmm_t and imq_qmm_t_noalloc */
     IMQ_ENTRY_QGEMM = 1,   /* imq_qgemm */
     IMQ_ENTRY_QGEMV = 2,   /* imq_qgemv */
-    IMQ_ENTRY_FUSED = 3,   /* imq_qmm_postscale / _gate_add (n = weight rows) */
+    IMQ_ENTRY_FUSED = 3,   /* imq_qmm_postscale / _gate_add (n = weight rows); imq_qmm_add runs the
+                              same kernel, past 128 rows by tiles that may differ */
     IMQ_ENTRY_SWIGLU = 4   /* imq_qmm_swiglu (n = 2 * width: the gate and up rows it reads) */
 } imq_entry;
 
 typedef enum imq_kernel {
     IMQ_KERNEL_QGEMV = 0,    /* register dequant, fp32 dot products, no matrix cores */
     IMQ_KERNEL_FEW_ROW = 1,  /* weight-streaming matrix-core kernel, 16 weight rows per workgroup */
-    IMQ_KERNEL_TILE = 2,     /* MFMA tiles, activations staged by direct buffer->LDS loads
-                                (K % 256 == 0) */
-    IMQ_KERNEL_TILE_REG = 3  /* MFMA tiles, activations staged through registers (other K) */
+    IMQ_KERNEL_TILE = 2,     /* MFMA tiles, activations staged by direct buffer->LDS loads */
+    IMQ_KERNEL_TILE_REG = 3  /* MFMA tiles, activations staged through registers: a K that is not
+                                a multiple of 256, up to 1700, where its tiles fit better, and
+                                operands past 32-bit offsets */
 } imq_kernel;
 
 typedef struct imq_plan {

@@ -47,7 +47,7 @@ hipError_t launch_qgemm(const uint32_t*, const void*, const void*, const void*, 
   return hipErrorNoDevice;
 }
 size_t qgemm_split_bytes(int, int, int, bool) { return 0; }
-QgemmPlan qgemm_plan(int k, int n, int m, bool, bool, int, bool) {
+QgemmPlan qgemm_plan(int k, int n, int m, bool, bool) {
   return QgemmPlan{qgemm_big_supported(k, n, m), 128, 1, 0, 256};
 }
 bool qgemm_big_supported(int k, int n, int m) {

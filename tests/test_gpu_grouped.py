@@ -4,8 +4,9 @@ Each product of a group keeps its own rows, weights and output stage, and no
 stage but the gated residual add may split K: q, k and v equal imq_qgemm bit
 for bit, and the residual after both halves equals the same products and glue
 within the reordering of their fp32 sums (MAE 1e-3, normwise 1e-2).  Row counts
-put the tiles' edges in every place: one tile for both, a text part larger than
-the image part, single rows, and a K long enough for the MLP-outs to split.
+take the 128-row tiles (128 and 256 columns; the taller ones are in
+test_gpu_group_plans.py) through their edges: one tile for both, a text part larger
+than the image part, single rows, and a K long enough for the MLP-outs to split.
 """
 
 from __future__ import annotations
