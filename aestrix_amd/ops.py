@@ -332,7 +332,8 @@ def qmm_gate_add(x, w, scales, biases, residual: torch.Tensor, gate: torch.Tenso
 # Host ids past this many are copied to the device in one piece instead: that costs
 # about the same at any count, the arguments one launch per 768 (2560 wide, us a
 # call, copied / as arguments: 30 ids 31.9 / 13.5, 3072 38.1 / 26.4, 4608 38.4 / 35.1,
-# 6144 39.5 / 42.8, 12288 46.9 / 74.5).
+# 6144 39.5 / 42.8, 12288 46.9 / 74.5).  A stream under capture takes arguments at any
+# count: it refuses the copy.
 MAX_ARG_ROWS = 6 * 768
 
 
@@ -346,7 +347,8 @@ def dequantize_rows(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
     n, k = _check_weight(w, scales, biases, group_size, bits)
     _require(rows.dim() == 1 and rows.dtype in (torch.int32, torch.int64), "rows: 1-D integer ids")
     idx, count = w.get_device(), rows.numel()
-    host = rows.device.type == "cpu" and count <= MAX_ARG_ROWS
+    host = rows.device.type == "cpu" and (
+        count <= MAX_ARG_ROWS or run_on(idx, torch.cuda.is_current_stream_capturing))
     if host:
         ids = rows.to(torch.int64).contiguous()
         if ids.data_ptr() % 8:  # ids in the middle of a byte buffer

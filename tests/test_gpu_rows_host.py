@@ -73,3 +73,22 @@ def test_host_ids_in_the_middle_of_a_byte_buffer():
         ids = torch.frombuffer(buf, dtype=torch.int64, offset=off)
         print(f"rows by host ids {ids.data_ptr() % 8} bytes past a multiple of 8", flush=True)
         assert torch.equal(imq.dequantize_rows(w, s, b, ids), want[:40])
+
+
+def test_more_host_ids_than_arguments_pay_for_are_captured():
+    n, k, count = 300, 64, ops.MAX_ARG_ROWS + 900
+    _, w, s, b = synth.to_device(synth.make_problem(1, n, k, seed=8))
+    ids = torch.randint(0, n, (count,), generator=torch.Generator().manual_seed(3))
+    want = imq.dequantize(w, s, b)[ids.cuda()]
+    out = torch.empty_like(want)
+    imq.dequantize_rows(w, s, b, ids, out=out)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=side):
+        imq.dequantize_rows(w, s, b, ids, out=out)
+    for _ in range(3):
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
